@@ -3198,7 +3198,8 @@ int run_bidir(hipStream_t st, const float* X, const float* Y, int64_t m, int64_t
         // this chunk's split copy of X (the sweeps take the copy from the chunk's first row)
         if (split && cp.x_chunked)
             if (int rc = copy_rows(false, xb, rows, xsplit)) return rc;
-        const float* SXc = !split ? SX : (cp.x_chunked ? xsplit : SX + xb * ld);
+        // (the wide pass gathers queued rows by their number within the chunk, whatever the sweep reads)
+        const float* SXc = cp.x_chunked ? xsplit : SX + xb * ld;
         // floors of this chunk's column lists: the caller's, and after the first chunk the running lists' k-th
         // values (a chunk's lists then only keep what can enter the merged lists)
         const double* cfloor = wide.col_floor;
@@ -3335,7 +3336,7 @@ int run_bidir(hipStream_t st, const float* X, const float* Y, int64_t m, int64_t
             // this chunk's split copy of Y (from its first row; a resident side's copy is whole)
             if (split && cp.y_chunked && !q8.y_ready)
                 if (int rc = copy_rows(true, yb, rows, ysplit)) return rc;
-            const float* SYc = !split ? SY : ((cp.y_chunked && !q8.y_ready) ? ysplit : SY + yb * ld);
+            const float* SYc = (cp.y_chunked && !q8.y_ready) ? ysplit : SY + yb * ld;
             // the rows' shared thresholds start at -inf, or at the caller's column floors
             const dim3 tgrid((unsigned)((rows + 255) / 256 < 4096 ? (rows + 255) / 256 : 4096));
             if (wide.col_floor)

@@ -151,6 +151,39 @@ def test_l2sq_chunked_sides_and_ties(cuda, m, n, d, k, integer, precision):
     assert_l2sq_certificate(st, l2sq_certificate_bounds(X, Y, p, q, qb, db))
 
 
+@pytest.mark.parametrize("side", ["x", "y"])
+@pytest.mark.parametrize("d", [5, 256])
+@pytest.mark.parametrize("precision", ["fp32", "bf16x3", "int8x3"])
+def test_l2sq_wide_pass_in_a_later_chunk(cuda, side, d, precision):
+    # 150 points of a side's second internal chunk (rows past 65536) sit with 150 of the other side within 1e-4 of one
+    # point, next to each other: their lists cannot be separated and go to the wide pass, which gathers its rows and
+    # reads its candidates by their number within the chunk
+    rng = np.random.default_rng(d)
+    big, small, k = 65536 + 400, 600, 2
+    base = rng.standard_normal(d).astype(np.float32)
+    L = (3.0 * rng.standard_normal((big, d))).astype(np.float32)
+    S = (3.0 * rng.standard_normal((small, d))).astype(np.float32)
+    L[65536 + 100:65536 + 250] = (base + 1e-4 * rng.standard_normal((150, d))).astype(np.float32)
+    S[200:350] = (base + 1e-4 * rng.standard_normal((150, d))).astype(np.float32)
+    X, Y = (L, S) if side == "x" else (S, L)
+    p = (X.astype(np.float64) ** 2).sum(1)
+    q = (Y.astype(np.float64) ** 2).sum(1)
+    orv, ori, ocv, oci, _ = oracle.l2sq_scan(X, Y, p, q, -p, -q, k, 2.0)
+    _lib.profile_reset()
+    _lib.profile_enable(True)
+    try:
+        rv, ri, cv, ci, _ = pricing_l2sq(*_to(cuda, X, Y, p, q, -p, -q), k, stats=False, precision=precision)
+        torch.cuda.synchronize()
+        swept = _lib.profile_query("l2sq_wide_rows")[1] + _lib.profile_query("l2sq_wide_columns")[1]
+    finally:
+        _lib.profile_enable(False)
+    np.testing.assert_array_equal(ri.cpu().numpy(), ori)
+    np.testing.assert_array_equal(rv.cpu().numpy(), orv)
+    np.testing.assert_array_equal(ci.cpu().numpy(), oci)
+    np.testing.assert_array_equal(cv.cpu().numpy(), ocv)
+    assert swept > 0
+
+
 @pytest.mark.parametrize("precision", ["fp32", "bf16x3", "int8x3"])
 @pytest.mark.parametrize("copies", [400, 1500])
 def test_l2sq_dense_near_ties_resolved_exactly(cuda, precision, copies):
