@@ -508,6 +508,49 @@ def test_norm_fused_sweep_ragged_rows_and_wide_features(cuda, kind, m, n, d, k):
 
 
 @pytest.mark.parametrize("kind", [0, 1, 2])
+@pytest.mark.parametrize("m,n,d,k", [
+    (1, 1, 1, 1), (2, 513, 3, 2), (257, 255, 4, 4), (300, 256, 5, 16), (513, 1, 7, 2), (200, 530, 8, 32),
+    (256, 700, 9, 2), (140, 511, 16, 17), (90, 300, 17, 1), (150, 260, 24, 8), (70, 800, 25, 2), (90, 257, 32, 16),
+    (70, 300, 33, 2), (129, 270, 48, 4), (64, 513, 49, 2), (50, 260, 63, 16), (40, 260, 64, 2), (40, 300, 95, 2),
+    (30, 520, 96, 32), (33, 257, 97, 2), (20, 300, 128, 16), (25, 260, 129, 2), (20, 130, 160, 4)])
+def test_norm_sweep_widths_tiles_and_list_lengths(cuda, kind, m, n, d, k):
+    """Every register width with whole and partial feature groups, one-column and partial tiles, odd columns of a step,
+    lists longer than a side and of each workgroup shape, against the oracle (costs and scores are exact)."""
+    rng = np.random.default_rng(m + 5 * n + 11 * d + kind)
+    X = rng.normal(0.0, 1.0, (m, d)).astype(np.float32)
+    Y = rng.normal(0.0, 1.0, (n, d)).astype(np.float32)
+    Y[n // 2] = Y[0]                                   # tied costs
+    f, g = rng.normal(0.5, 0.3, m) * d ** 0.5, rng.normal(0.5, 0.3, n) * d ** 0.5
+    g[n // 2] = g[0]
+    orv, ori, ocv, oci, ost = oracle.norm_scan(X, Y, f, g, k, kind)
+    rv, ri, cv, ci, st = pricing_norm(*_to(cuda, X, Y, f, g), k, kind)
+    np.testing.assert_array_equal(ri.cpu().numpy(), ori)
+    np.testing.assert_array_equal(rv.cpu().numpy(), orv)
+    np.testing.assert_array_equal(ci.cpu().numpy(), oci)
+    np.testing.assert_array_equal(cv.cpu().numpy(), ocv)
+    _assert_stats(st, ost)
+
+
+@pytest.mark.parametrize("kind,d", [(0, 3), (1, 8), (2, 20), (0, 32)])
+def test_norm_two_rows_per_thread_agree_with_one(cuda, kind, d):
+    """Large sides with short lists run two rows per thread and, with both directions, column lists on the row sweep;
+    lists of 8 run one row per thread and two sweeps. The first two entries of the long lists are the short ones, and the
+    certificates differ by the order of their sums (1e-9: fp64 sums of per-tile fp32 sums of the same terms)."""
+    g0 = torch.Generator(device=cuda).manual_seed(90 + d)
+    m, n = 70001, 8300
+    X = torch.rand(m, d, generator=g0, device=cuda)
+    Y = torch.rand(n, d, generator=g0, device=cuda)
+    f = 0.2 * d ** 0.5 * torch.rand(m, generator=g0, device=cuda, dtype=torch.float64)
+    g = 0.2 * torch.rand(n, generator=g0, device=cuda, dtype=torch.float64)
+    short, long = pricing_norm(X, Y, f, g, 2, kind), pricing_norm(X, Y, f, g, 8, kind)
+    for a, b in zip(short[:4], long[:4]):
+        assert torch.equal(a, b[:, :2])
+    a, b = short[4].cpu().numpy(), long[4].cpu().numpy()
+    assert a[2] == b[2] and a[3] == b[3] and a[4] == b[4]
+    np.testing.assert_allclose(a[:2], b[:2], rtol=1e-9)
+
+
+@pytest.mark.parametrize("kind", [0, 1, 2])
 @pytest.mark.parametrize("k,grid", [(2, False), (1, False), (2, True)])
 def test_norm_fused_columns_overflow_and_two_sweep_paths_agree(cuda, kind, k, grid):
     """k <= 2 bidirectional calls evaluate each pair once and collect the column lists through the candidate buffer.
