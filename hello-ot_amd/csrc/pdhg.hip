@@ -13,19 +13,21 @@
 //   target order (slot k): edges sorted by target, ascending caller edge id within a target, so target t owns
 //     [off[n+t]-e, off[n+t+1]-e). Arrays: row_t, cs_t, x_t, ax_t, px_t.
 // Both copies receive identical operands in identical order and therefore stay bit-identical.
-// Per node (sources then targets): scale, bs, ns, y, ay, py, dy; td = y / ns for targets and sd = y / ns for
-// sources (the value the current iteration's primal step used).
+// Per node (sources then targets): scale, bs, ns, y, ay, py, dy, and dual = y / ns in two buffers: an iteration reads
+// the duals of one and writes the next ones to the other.
 //
-// One iteration = source pass + target pass (the restatement's two loops):
-//   source pass: per source node, its edges' PDHG step and reflection, their iterates (Halpern), and the node's
+// One iteration is one launch: the restatement's two loops (source nodes, then target nodes) both start from the duals
+// of the previous iteration, so with the next duals going to another buffer nothing orders them, and the workgroups of
+// both sides run together:
+//   source side: per source node, its edges' PDHG step and reflection, their iterates (Halpern), and the node's
 //                dual from the in-order sum of the reflections;
-//   target pass: per target node, the same steps for its edges from the mirrored state and the source duals sd,
-//                and the target dual from its in-order sum.
+//   target side: per target node, the same steps for its edges from the mirrored state, and its dual from its
+//                in-order sum.
 // Each side runs in one of two shapes, chosen per solve from the side's largest degree: G-lane groups per node
 // (lanes sum in edge order through shuffles) when every node fits in one chunk of the group, else node blocks
 // (edge-parallel steps, then one thread per node sums its reflections in edge order from LDS). Both are
 // bit-identical to a sequential sum.
-// The only gathers are of node values (sd, td). Scalars read back to the host only at evaluations and checkpoints.
+// The only gathers are of duals. Scalars read back to the host only at evaluations and checkpoints.
 //
 // Node numbering: on large problems (at least HELLOOT_PDHG_REORDER nodes, default 2^20, where the duals outgrow
 // an XCD's L2) the nodes are renumbered inside the solve so that nodes joined by many edges get nearby numbers:
@@ -67,7 +69,8 @@ struct Pdhg {
     uint16_t *g16_s, *g16_t;
     int32_t *gbase_s, *gbase_t;
     // nodes
-    double *scale, *bs, *ns, *y, *ay, *py, *dy, *td, *sd;
+    double *scale, *bs, *ns, *y, *ay, *py, *dy;
+    double* dual[2];
     int32_t *deg, *off, *eid;
     // node numbering (map_s / map_t: internal number of a caller source / target, or null for the identity;
     // inv: caller node of an internal node, sources then targets) and its scratch
@@ -117,8 +120,7 @@ void pdhg_layout(A& a, int64_t n, int64_t nt, int64_t e, size_t sort_tmp, size_t
     P.ay = a.template take<double>(nodes);
     P.py = a.template take<double>(nodes);
     P.dy = a.template take<double>(nodes);
-    P.td = a.template take<double>(nt);
-    P.sd = a.template take<double>(n);
+    P.dual[0] = a.template take<double>(nodes);
     P.deg = a.template take<int32_t>(nodes + 1);
     P.off = a.template take<int32_t>(nodes + 1);
     P.eid = a.template take<int32_t>(2 * e);
@@ -136,6 +138,7 @@ void pdhg_layout(A& a, int64_t n, int64_t nt, int64_t e, size_t sort_tmp, size_t
     P.odeg = a.template take<int32_t>(nodes);
     P.ov = a.template take<uint32_t>(nodes);
     P.osum = a.template take<unsigned long long>(nodes);
+    P.dual[1] = reinterpret_cast<double*>(P.osum);  // the numbering is done before the first iteration writes it
     P.okeys_in = a.template take<unsigned long long>(side);
     P.okeys_out = a.template take<unsigned long long>(side);
     P.osort_tmp = a.template take<char>(osort_tmp > 0 ? osort_tmp : 1);
@@ -330,11 +333,11 @@ __global__ void k_scan(const int32_t* __restrict__ deg, int64_t nodes, int32_t* 
 }
 
 __global__ void k_node_setup(const int32_t* __restrict__ deg, const double* __restrict__ b,
-                             const double* __restrict__ y0, const int32_t* __restrict__ inv, int64_t nodes, int64_t n,
+                             const double* __restrict__ y0, const int32_t* __restrict__ inv, int64_t nodes,
                              double bound, double objective, double variable, double* __restrict__ scale,
                              double* __restrict__ bs, double* __restrict__ ns, double* __restrict__ y,
                              double* __restrict__ ay, double* __restrict__ py, double* __restrict__ dy,
-                             double* __restrict__ td) {
+                             double* __restrict__ dual) {
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < nodes; i += (int64_t)gridDim.x * blockDim.x) {
         const int64_t o = inv ? inv[i] : i;  // the caller's number of internal node i
         const double sc = sqrt((double)(deg[i] > 1 ? deg[i] : 1));
@@ -347,7 +350,7 @@ __global__ void k_node_setup(const int32_t* __restrict__ deg, const double* __re
         y[i] = a;
         py[i] = a;
         dy[i] = 0.0;
-        if (i >= n) td[i - n] = a / nsv;
+        dual[i] = a / nsv;
     }
 }
 
@@ -539,107 +542,82 @@ __device__ inline double group_ordered_sum(double running, double value, int cou
     return running;
 }
 
-// Source pass: a G-lane group per source node (the restatement's first loop, solver.cpp:210-251 order).
-// A chunk covers G*U edges: lane g owns edges g, g+G, ..., g+(U-1)G of the chunk, all loaded before any sum.
-template <int G, int U, bool CHECKPOINT, bool STORE>
-__global__ __launch_bounds__(256) void k_source_pass(const Pdhg P, double primal_step, double dual_step,
-                                                     double halpern) {
-    const double keep = 1.0 - halpern;
-    const int g = threadIdx.x % G;
-    const int64_t stride = (int64_t)gridDim.x * (blockDim.x / G);
-    for (int64_t i = (int64_t)blockIdx.x * (blockDim.x / G) + threadIdx.x / G; i < P.n; i += stride) {
-        const int32_t k0 = P.off[i], k1 = P.off[i + 1];
-        const double yi = P.y[i], nsi = P.ns[i];
-        const double source_dual = yi / nsi;
-        double sum = 0.0;
-        for (int32_t base = k0; base < k1; base += G * U) {
-            double r[U];
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const int32_t p = base + u * G + g;
-                r[u] = 0.0;
-                if (p < k1) {
-                    const double at = source_dual + P.td[P.col[p]];
-                    const double xj = P.x[p];
-                    const double pxj = fmax(xj - primal_step * (P.cs[p] - at), 0.0);
-                    r[u] = 2.0 * pxj - xj;
-                    if (STORE) P.px[p] = pxj;
-                    if (CHECKPOINT) P.dx[p] = r[u] - xj;
-                    P.x[p] = halpern * r[u] + keep * P.ax[p];
-                }
-            }
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const int32_t left = k1 - (base + u * G);
-                if (left > 0) sum = group_ordered_sum<G>(sum, r[u], left < G ? left : G);
-            }
-        }
-        if (g == 0) {
-            P.sd[i] = source_dual;
-            const double pyi = yi - dual_step * (sum / nsi - P.bs[i]);
-            const double refl = 2.0 * pyi - yi;
-            if (STORE) P.py[i] = pyi;
-            if (CHECKPOINT) P.dy[i] = refl - yi;
-            P.y[i] = halpern * refl + keep * P.ay[i];
-        }
-    }
+// One side of an iteration: its nodes [first, first + count) of the node arrays, its edges in its own order (the
+// arrays of Pdhg's source or target half), and the first node of the other side, whose duals its edges gather.
+struct Side {
+    int64_t first, count, other;
+    int32_t ebase;          // position of the side's first edge in off
+    const int32_t* gidx;    // the other side's node of each edge
+    const double *cs, *ax;
+    double *x, *px, *dx;    // dx: the source side alone (the checkpoint deltas of the edges)
+    const uint8_t* loc;
+    const uint16_t* g16;
+    const int32_t* gbase;
+};
+
+// one edge's step: the PDHG point, its reflection and the Halpern iterate (solver.cpp:210-251 order)
+template <bool SOURCE, bool CHECKPOINT, bool STORE>
+__device__ __forceinline__ double edge_step(const Side& sd, int32_t p, double own, double other, double primal_step,
+                                            double halpern, double keep) {
+    const double at = SOURCE ? own + other : other + own;
+    const double xj = sd.x[p];
+    const double pxj = fmax(xj - primal_step * (sd.cs[p] - at), 0.0);
+    const double r = 2.0 * pxj - xj;
+    if (STORE) sd.px[p] = pxj;
+    if (CHECKPOINT && SOURCE) sd.dx[p] = r - xj;
+    sd.x[p] = halpern * r + keep * sd.ax[p];
+    return r;
 }
 
-// Target pass: a G-lane group per target node recomputes its edges' steps from the target-order mirror (the
-// operands are those the source pass used: sd of this iteration, td before this update) and updates the dual.
-template <int G, int U, bool CHECKPOINT, bool STORE>
-__global__ __launch_bounds__(256) void k_target_pass(const Pdhg P, double primal_step, double dual_step,
-                                                     double halpern) {
-    const double keep = 1.0 - halpern;
-    const int g = threadIdx.x % G;
-    const int64_t stride = (int64_t)gridDim.x * (blockDim.x / G);
-    for (int64_t t = (int64_t)blockIdx.x * (blockDim.x / G) + threadIdx.x / G; t < P.nt; t += stride) {
-        const int64_t i = P.n + t;
-        const int32_t k0 = P.off[i] - (int32_t)P.e, k1 = P.off[i + 1] - (int32_t)P.e;
-        const double target_dual = P.td[t];
-        double sum = 0.0;
-        for (int32_t base = k0; base < k1; base += G * U) {
-            double r[U];
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const int32_t k = base + u * G + g;
-                r[u] = 0.0;
-                if (k < k1) {
-                    const double at = P.sd[P.row_t[k]] + target_dual;
-                    const double xj = P.x_t[k];
-                    const double pxj = fmax(xj - primal_step * (P.cs_t[k] - at), 0.0);
-                    r[u] = 2.0 * pxj - xj;
-                    if (STORE) P.px_t[k] = pxj;
-                    P.x_t[k] = halpern * r[u] + keep * P.ax_t[k];
-                }
-            }
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const int32_t left = k1 - (base + u * G);
-                if (left > 0) sum = group_ordered_sum<G>(sum, r[u], left < G ? left : G);
-            }
-        }
-        if (g == 0) {
-            const double yi = P.y[i], nsi = P.ns[i];
-            const double pyi = yi - dual_step * (sum / nsi - P.bs[i]);
-            const double refl = 2.0 * pyi - yi;
-            if (STORE) P.py[i] = pyi;
-            if (CHECKPOINT) P.dy[i] = refl - yi;
-            const double yn = halpern * refl + keep * P.ay[i];
-            P.y[i] = yn;
-            P.td[t] = yn / nsi;
-        }
-    }
+// a node's update from the sum of its reflections
+template <bool CHECKPOINT, bool STORE>
+__device__ __forceinline__ void node_step(const Pdhg& P, int64_t i, double sum, double dual_step, double halpern,
+                                          double keep, double* __restrict__ next) {
+    const double yi = P.y[i], nsi = P.ns[i];
+    const double pyi = yi - dual_step * (sum / nsi - P.bs[i]);
+    const double refl = 2.0 * pyi - yi;
+    if (STORE) P.py[i] = pyi;
+    if (CHECKPOINT) P.dy[i] = refl - yi;
+    const double yn = halpern * refl + keep * P.ay[i];
+    P.y[i] = yn;
+    next[i] = yn / nsi;
 }
 
-// Node-block passes: a workgroup owns `npb` consecutive nodes of one side and their edges (contiguous in that side's
-// order). Edges are processed EB at a time: every thread computes edge steps (coalesced streams, one gather of the
-// other side's dual), the reflections go to LDS, and then one thread per node adds its edges' reflections in edge
-// order from LDS, carrying its running sum across the rounds. Same operations, operands and order as the
-// lane-group passes above, so the iterates are bit-identical; the work per workgroup follows the edges, not the
-// node count, and a node's fold is a run of LDS reads instead of lane shuffles.
-constexpr int EB = 2048;  // edges per round
-constexpr int PT = 256;   // threads per workgroup (also the largest npb)
+constexpr int EB = 2048;  // edges per round of a node block
+constexpr int PT = 256;   // threads per workgroup (also the most nodes of a node block)
+
+// Lane groups: a G-lane group per node (block `block` of the side). A chunk covers G*U edges: lane g owns edges g, g+G,
+// ..., g+(U-1)G of the chunk, all loaded before any sum.
+template <int G, int U, bool SOURCE, bool CHECKPOINT, bool STORE>
+__device__ __forceinline__ void group_pass(const Pdhg& P, const Side& sd, int64_t block, const double* __restrict__ cur,
+                                           double* __restrict__ next, double primal_step, double dual_step,
+                                           double halpern) {
+    const double keep = 1.0 - halpern;
+    const int g = threadIdx.x % G;
+    const int64_t t = block * (PT / G) + threadIdx.x / G;
+    if (t >= sd.count) return;
+    const int64_t i = sd.first + t;
+    const int32_t k0 = P.off[i] - sd.ebase, k1 = P.off[i + 1] - sd.ebase;
+    const double own = cur[i];
+    double sum = 0.0;
+    for (int32_t base = k0; base < k1; base += G * U) {
+        double r[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int32_t p = base + u * G + g;
+            r[u] = 0.0;
+            if (p < k1)
+                r[u] = edge_step<SOURCE, CHECKPOINT, STORE>(sd, p, own, cur[sd.other + sd.gidx[p]], primal_step, halpern,
+                                                            keep);
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int32_t left = k1 - (base + u * G);
+            if (left > 0) sum = group_ordered_sum<G>(sum, r[u], left < G ? left : G);
+        }
+    }
+    if (g == 0) node_step<CHECKPOINT, STORE>(P, i, sum, dual_step, halpern, keep, next);
+}
 
 // sum + v[a] + v[a+1] + ... + v[b-1], added one by one in that order; the LDS reads go out eight at a time so that
 // a long node waits for one read latency per eight values rather than per value.
@@ -656,113 +634,85 @@ __device__ __forceinline__ double fold_in_order(const double* v, int a, int b, d
     return sum;
 }
 
-template <bool CHECKPOINT, bool STORE>
-__global__ __launch_bounds__(PT) void k_source_block(const Pdhg P, double primal_step, double dual_step,
-                                                     double halpern, int npb) {
-    __shared__ double sr[EB];
-    __shared__ double sdl[PT];
-    __shared__ int32_t soff[PT + 1];
+struct BlockLds {
+    double refl[EB];
+    double dual[PT];
+    int32_t off[PT + 1];
+};
+
+// Node blocks: a workgroup owns `npb` consecutive nodes of one side and their edges (contiguous in that side's order).
+// Edges are processed EB at a time: every thread computes edge steps (coalesced streams, one gather of the other side's
+// dual), the reflections go to LDS, and then one thread per node adds its edges' reflections in edge order from LDS,
+// carrying its running sum across the rounds. Same operations, operands and order as the lane groups, so the iterates
+// are bit-identical; the work per workgroup follows the edges, not the node count, and a node's fold is a run of LDS
+// reads instead of lane shuffles.
+template <bool SOURCE, bool CHECKPOINT, bool STORE>
+__device__ __forceinline__ void block_pass(const Pdhg& P, const Side& sd, int64_t block, int npb,
+                                           const double* __restrict__ cur, double* __restrict__ next,
+                                           double primal_step, double dual_step, double halpern, BlockLds& lds) {
     const int tid = threadIdx.x;
-    const int64_t n0 = (int64_t)blockIdx.x * npb;
-    const int nn = (int)(P.n - n0 < npb ? P.n - n0 : npb);
+    const int64_t n0 = sd.first + block * npb;
+    const int64_t left = sd.count - block * npb;
+    const int nn = (int)(left < npb ? left : npb);
     const double keep = 1.0 - halpern;
-    double yi = 0.0, nsi = 1.0;
-    if (tid < nn) {
-        yi = P.y[n0 + tid];
-        nsi = P.ns[n0 + tid];
-        sdl[tid] = yi / nsi;
-    }
-    for (int t = tid; t <= nn; t += PT) soff[t] = P.off[n0 + t];
+    const double* const other = cur + sd.other;
+    if (tid < nn) lds.dual[tid] = cur[n0 + tid];
+    for (int t = tid; t <= nn; t += PT) lds.off[t] = P.off[n0 + t] - sd.ebase;
+    const int32_t gb = sd.gbase[block];  // uniform: 16-bit gather offsets, or -1 for 4-byte numbers
     __syncthreads();
-    const int32_t e0 = soff[0], e1 = soff[nn];
-    const int32_t k0 = tid < nn ? soff[tid] : 0, k1 = tid < nn ? soff[tid + 1] : 0;
+    const int32_t e0 = lds.off[0], e1 = lds.off[nn];
+    const int32_t k0 = tid < nn ? lds.off[tid] : 0, k1 = tid < nn ? lds.off[tid + 1] : 0;
     double sum = 0.0;
-    const int32_t gb = P.gbase_s[blockIdx.x];  // uniform: 16-bit gather offsets, or -1 for 4-byte numbers
-    // edge p (slot q of the round) with its target c
-    auto step = [&](int32_t p, int q, int32_t c) {
-        const double at = sdl[P.loc_s[p]] + P.td[c];
-        const double xj = P.x[p];
-        const double pxj = fmax(xj - primal_step * (P.cs[p] - at), 0.0);
-        const double r = 2.0 * pxj - xj;
-        if (STORE) P.px[p] = pxj;
-        if (CHECKPOINT) P.dx[p] = r - xj;
-        P.x[p] = halpern * r + keep * P.ax[p];
-        sr[q] = r;
-    };
     for (int32_t base = e0; base < e1; base += EB) {
         const int len = e1 - base < EB ? e1 - base : EB;
-        if (gb >= 0) {
-            for (int q = tid; q < len; q += PT) step(base + q, q, gb + (int32_t)P.g16_s[base + q]);
-        } else {
-            for (int q = tid; q < len; q += PT) step(base + q, q, P.col[base + q]);
+        for (int q = tid; q < len; q += PT) {
+            const int32_t p = base + q;
+            const int32_t c = gb >= 0 ? gb + (int32_t)sd.g16[p] : sd.gidx[p];
+            lds.refl[q] = edge_step<SOURCE, CHECKPOINT, STORE>(sd, p, lds.dual[sd.loc[p]], other[c], primal_step, halpern,
+                                                               keep);
         }
         __syncthreads();
-        sum = fold_in_order(sr, (k0 > base ? k0 : base) - base, (k1 < base + len ? k1 : base + len) - base, sum);
+        sum = fold_in_order(lds.refl, (k0 > base ? k0 : base) - base, (k1 < base + len ? k1 : base + len) - base, sum);
         __syncthreads();
     }
-    if (tid < nn) {
-        const int64_t i = n0 + tid;
-        P.sd[i] = sdl[tid];
-        const double pyi = yi - dual_step * (sum / nsi - P.bs[i]);
-        const double refl = 2.0 * pyi - yi;
-        if (STORE) P.py[i] = pyi;
-        if (CHECKPOINT) P.dy[i] = refl - yi;
-        P.y[i] = halpern * refl + keep * P.ay[i];
+    if (tid < nn) node_step<CHECKPOINT, STORE>(P, n0 + tid, sum, dual_step, halpern, keep, next);
+}
+
+// How one side runs: lane groups of U edges per lane (u > 0), or node blocks (u = 0); its workgroups.
+struct SidePlan {
+    int u, npb;
+    int64_t blocks;
+};
+
+constexpr int GL = 8;  // lanes per group
+
+// One PDHG iteration: workgroups [0, src.blocks) run the source side, the rest the target side. Small problems are
+// bound by the latency of a launch and of each pass's chain of dependent loads (offsets, edges, gathered dual, fold),
+// which the two sides now share: 4096 nodes a side and 61 thousand edges take 10.0 us an iteration, as two dependent
+// launches they took 11.3. Large ones stream the edge state (524288 a side, 12.5 million edges: 318 us, before 324).
+template <bool CHECKPOINT, bool STORE>
+__global__ __launch_bounds__(PT) void k_iteration(const Pdhg P, SidePlan src, SidePlan tgt, const double* __restrict__ cur,
+                                                  double* __restrict__ next, double ps, double ds, double h) {
+    __shared__ BlockLds lds;
+    const int64_t b = blockIdx.x;
+    if (b < src.blocks) {
+        const Side sd{0, P.n, P.n, 0, P.col, P.cs, P.ax, P.x, P.px, P.dx, P.loc_s, P.g16_s, P.gbase_s};
+        if (src.u == 0) block_pass<true, CHECKPOINT, STORE>(P, sd, b, src.npb, cur, next, ps, ds, h, lds);
+        else if (src.u == 1) group_pass<GL, 1, true, CHECKPOINT, STORE>(P, sd, b, cur, next, ps, ds, h);
+        else if (src.u == 2) group_pass<GL, 2, true, CHECKPOINT, STORE>(P, sd, b, cur, next, ps, ds, h);
+        else group_pass<GL, 4, true, CHECKPOINT, STORE>(P, sd, b, cur, next, ps, ds, h);
+    } else {
+        const int64_t bt = b - src.blocks;
+        const Side sd{P.n, P.nt, 0, (int32_t)P.e, P.row_t, P.cs_t, P.ax_t, P.x_t, P.px_t, nullptr, P.loc_t, P.g16_t,
+                      P.gbase_t};
+        if (tgt.u == 0) block_pass<false, CHECKPOINT, STORE>(P, sd, bt, tgt.npb, cur, next, ps, ds, h, lds);
+        else if (tgt.u == 1) group_pass<GL, 1, false, CHECKPOINT, STORE>(P, sd, bt, cur, next, ps, ds, h);
+        else if (tgt.u == 2) group_pass<GL, 2, false, CHECKPOINT, STORE>(P, sd, bt, cur, next, ps, ds, h);
+        else group_pass<GL, 4, false, CHECKPOINT, STORE>(P, sd, bt, cur, next, ps, ds, h);
     }
 }
 
-template <bool CHECKPOINT, bool STORE>
-__global__ __launch_bounds__(PT) void k_target_block(const Pdhg P, double primal_step, double dual_step,
-                                                     double halpern, int npb) {
-    __shared__ double sr[EB];
-    __shared__ double tdl[PT];
-    __shared__ int32_t soff[PT + 1];
-    const int tid = threadIdx.x;
-    const int64_t t0 = (int64_t)blockIdx.x * npb;
-    const int nn = (int)(P.nt - t0 < npb ? P.nt - t0 : npb);
-    const double keep = 1.0 - halpern;
-    if (tid < nn) tdl[tid] = P.td[t0 + tid];
-    for (int t = tid; t <= nn; t += PT) soff[t] = P.off[P.n + t0 + t] - (int32_t)P.e;
-    __syncthreads();
-    const int32_t e0 = soff[0], e1 = soff[nn];
-    const int32_t k0 = tid < nn ? soff[tid] : 0, k1 = tid < nn ? soff[tid + 1] : 0;
-    double sum = 0.0;
-    const int32_t gb = P.gbase_t[blockIdx.x];  // uniform: 16-bit gather offsets, or -1 for 4-byte numbers
-    // edge k (slot q of the round) with its source c
-    auto step = [&](int32_t k, int q, int32_t c) {
-        const double at = P.sd[c] + tdl[P.loc_t[k]];
-        const double xj = P.x_t[k];
-        const double pxj = fmax(xj - primal_step * (P.cs_t[k] - at), 0.0);
-        const double r = 2.0 * pxj - xj;
-        if (STORE) P.px_t[k] = pxj;
-        P.x_t[k] = halpern * r + keep * P.ax_t[k];
-        sr[q] = r;
-    };
-    for (int32_t base = e0; base < e1; base += EB) {
-        const int len = e1 - base < EB ? e1 - base : EB;
-        if (gb >= 0) {
-            for (int q = tid; q < len; q += PT) step(base + q, q, gb + (int32_t)P.g16_t[base + q]);
-        } else {
-            for (int q = tid; q < len; q += PT) step(base + q, q, P.row_t[base + q]);
-        }
-        __syncthreads();
-        sum = fold_in_order(sr, (k0 > base ? k0 : base) - base, (k1 < base + len ? k1 : base + len) - base, sum);
-        __syncthreads();
-    }
-    if (tid < nn) {
-        const int64_t i = P.n + t0 + tid;
-        const double yi = P.y[i], nsi = P.ns[i];
-        const double pyi = yi - dual_step * (sum / nsi - P.bs[i]);
-        const double refl = 2.0 * pyi - yi;
-        if (STORE) P.py[i] = pyi;
-        if (CHECKPOINT) P.dy[i] = refl - yi;
-        const double yn = halpern * refl + keep * P.ay[i];
-        P.y[i] = yn;
-        P.td[t0 + tid] = yn / nsi;
-    }
-}
-
-__global__ void k_restart(const Pdhg P) {
+__global__ void k_restart(const Pdhg P, double* __restrict__ dual) {
     const int64_t total = P.e > P.nodes ? P.e : P.nodes;
     for (int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; j < total; j += (int64_t)gridDim.x * blockDim.x) {
         if (j < P.e) {
@@ -777,7 +727,7 @@ __global__ void k_restart(const Pdhg P) {
             const double v = P.py[j];
             P.ay[j] = v;
             P.y[j] = v;
-            if (j >= P.n) P.td[j - P.n] = v / P.ns[j];
+            dual[j] = v / P.ns[j];
         }
     }
 }
@@ -797,16 +747,6 @@ inline unsigned grid_of(int64_t items) {
     return (unsigned)b;
 }
 
-inline unsigned group_grid(int64_t nodes, int g) {
-    int64_t b = (nodes + (256 / g) - 1) / (256 / g);
-    if (b > 65536) b = 65536;
-    if (b < 1) b = 1;
-    return (unsigned)b;
-}
-
-// Both passes run GL-lane groups with U edges per lane per chunk (U = 1, 2 or 4 from the side's mean degree).
-constexpr int GL = 8;
-
 inline int edges_per_lane(int64_t e, int64_t nodes) {
     const int64_t mean = (e + nodes - 1) / nodes;
     return mean <= GL ? 1 : (mean <= 12 ? 2 : 4);
@@ -819,56 +759,26 @@ inline int nodes_per_block(int64_t nodes) {
     return npb;
 }
 
-// How one side's pass runs: lane groups of U edges per lane (u > 0), or node blocks (u = 0). Lane groups when
-// every node of the side fits in one chunk of GL * U edges: each lane then holds at most U independent edges and
-// no group waits for a longer neighbour. Otherwise node blocks, whose work follows the edges (on the supports of
-// the HELLO levels, where degrees spread to several times their mean, they take 27-32% less time per iteration;
-// on uniform degree 16 the lane groups are 8% faster).
-struct SidePlan {
-    int u, npb;
-};
-
+// Lane groups (U = 1, 2 or 4 from the side's mean degree) when every node of the side fits in one chunk of GL * U
+// edges: each lane then holds at most U independent edges and no group waits for a longer neighbour. Otherwise node
+// blocks, whose work follows the edges (on the supports of the HELLO levels, where degrees spread to several times
+// their mean, they take 27-32% less time per iteration; on uniform degree 16 the lane groups are 8% faster).
 inline SidePlan side_plan(int64_t e, int64_t nodes, int max_degree) {
     const int u = edges_per_lane(e, nodes);
-    return SidePlan{max_degree <= GL * u ? u : 0, nodes_per_block(nodes)};
+    SidePlan sp{max_degree <= GL * u ? u : 0, nodes_per_block(nodes), 0};
+    const int per = sp.u == 0 ? sp.npb : PT / GL;
+    sp.blocks = (nodes + per - 1) / per;
+    return sp;
 }
 
-template <bool C, bool S>
-void launch_source(hipStream_t st, const Pdhg& P, const SidePlan& sp, double ps, double ds, double h) {
-    const dim3 grid(group_grid(P.n, GL)), block(256);
-    if (sp.u == 0)
-        hipLaunchKernelGGL((k_source_block<C, S>), dim3((unsigned)((P.n + sp.npb - 1) / sp.npb)), dim3(PT), 0, st, P,
-                           ps, ds, h, sp.npb);
-    else if (sp.u == 1) hipLaunchKernelGGL((k_source_pass<GL, 1, C, S>), grid, block, 0, st, P, ps, ds, h);
-    else if (sp.u == 2) hipLaunchKernelGGL((k_source_pass<GL, 2, C, S>), grid, block, 0, st, P, ps, ds, h);
-    else hipLaunchKernelGGL((k_source_pass<GL, 4, C, S>), grid, block, 0, st, P, ps, ds, h);
-}
-
-template <bool C, bool S>
-void launch_target(hipStream_t st, const Pdhg& P, const SidePlan& sp, double ps, double ds, double h) {
-    const dim3 grid(group_grid(P.nt, GL)), block(256);
-    if (sp.u == 0)
-        hipLaunchKernelGGL((k_target_block<C, S>), dim3((unsigned)((P.nt + sp.npb - 1) / sp.npb)), dim3(PT), 0, st, P,
-                           ps, ds, h, sp.npb);
-    else if (sp.u == 1) hipLaunchKernelGGL((k_target_pass<GL, 1, C, S>), grid, block, 0, st, P, ps, ds, h);
-    else if (sp.u == 2) hipLaunchKernelGGL((k_target_pass<GL, 2, C, S>), grid, block, 0, st, P, ps, ds, h);
-    else hipLaunchKernelGGL((k_target_pass<GL, 4, C, S>), grid, block, 0, st, P, ps, ds, h);
-}
-
-template <bool C, bool S>
-void launch_pair(hipStream_t st, const Pdhg& P, const SidePlan& src, const SidePlan& tgt, double ps, double ds,
-                 double h) {
-    launch_source<C, S>(st, P, src, ps, ds, h);
-    launch_target<C, S>(st, P, tgt, ps, ds, h);
-}
-
-// One PDHG iteration (source pass + target pass). px / py are stored only on major iterations: they are read
-// only by the evaluation that follows one.
-int launch_iteration(hipStream_t st, const Pdhg& P, const SidePlan& src, const SidePlan& tgt, bool checkpoint,
-                     bool major, double ps, double ds, double h) {
-    if (major) launch_pair<true, true>(st, P, src, tgt, ps, ds, h);
-    else if (checkpoint) launch_pair<true, false>(st, P, src, tgt, ps, ds, h);
-    else launch_pair<false, false>(st, P, src, tgt, ps, ds, h);
+// One PDHG iteration from the duals of `cur` to those of `next`. px / py are stored only on major iterations: they are
+// read only by the evaluation that follows one.
+int launch_iteration(hipStream_t st, const Pdhg& P, const SidePlan& src, const SidePlan& tgt, const double* cur,
+                     double* next, bool checkpoint, bool major, double ps, double ds, double h) {
+    const dim3 grid((unsigned)(src.blocks + tgt.blocks)), block(PT);
+    if (major) hipLaunchKernelGGL((k_iteration<true, true>), grid, block, 0, st, P, src, tgt, cur, next, ps, ds, h);
+    else if (checkpoint) hipLaunchKernelGGL((k_iteration<true, false>), grid, block, 0, st, P, src, tgt, cur, next, ps, ds, h);
+    else hipLaunchKernelGGL((k_iteration<false, false>), grid, block, 0, st, P, src, tgt, cur, next, ps, ds, h);
     HM_LAUNCH_CHECK("pdhg iteration");
     return HM_OK;
 }
@@ -1002,8 +912,8 @@ extern "C" int hm_pdhg_solve(void* stream, const int64_t* rows, const int64_t* c
     hipLaunchKernelGGL(k_target_setup, dim3(grid_of(e)), dim3(256), 0, st, P.eid, e, rows, cols, costs, x0, bound,
                        objective, variable, P);
     HM_LAUNCH_CHECK("k_target_setup");
-    hipLaunchKernelGGL(k_node_setup, dim3(grid_of(nodes)), dim3(256), 0, st, P.deg, masses, y0, P.inv, nodes, n, bound,
-                       objective, variable, P.scale, P.bs, P.ns, P.y, P.ay, P.py, P.dy, P.td);
+    hipLaunchKernelGGL(k_node_setup, dim3(grid_of(nodes)), dim3(256), 0, st, P.deg, masses, y0, P.inv, nodes, bound,
+                       objective, variable, P.scale, P.bs, P.ns, P.y, P.ay, P.py, P.dy, P.dual[0]);
     HM_LAUNCH_CHECK("k_node_setup");
     double weight = 1.0;
     if (!rescale) {
@@ -1025,6 +935,7 @@ extern "C" int hm_pdhg_solve(void* stream, const int64_t* rows, const int64_t* c
     int64_t count = 0, inner = 0, restarts = 0;
     double pobj = 0, dobj = 0, ap = 0, rp = 0, ad = 0, rd = 0, gap = 0;
     int64_t local_count = 0, local_inner = 0;
+    int at = 0;  // the dual buffer the next iteration reads
     const unsigned gr = grid_of(e > nodes ? e : nodes);
     const SidePlan src = side_plan(e, n, flag[1]), tgt = side_plan(e, nt, flag[2]);
     static_assert(PT <= 256, "a node's index within its block fits one byte");
@@ -1092,7 +1003,7 @@ extern "C" int hm_pdhg_solve(void* stream, const int64_t* rows, const int64_t* c
                 inner = 0;
                 last_trial_error = inf;
                 ++restarts;
-                hipLaunchKernelGGL(k_restart, dim3(gr), dim3(256), 0, st, P);
+                hipLaunchKernelGGL(k_restart, dim3(gr), dim3(256), 0, st, P, P.dual[at]);
                 HM_LAUNCH_CHECK("k_restart");
                 local_inner = 0;
             }
@@ -1105,7 +1016,10 @@ extern "C" int hm_pdhg_solve(void* stream, const int64_t* rows, const int64_t* c
         const bool checkpoint = major || is_restart;
         // px / py are read only by the evaluation that follows a major iteration
         prof_begin(st, "pdhg_iteration");
-        if (int rc = launch_iteration(st, P, src, tgt, checkpoint, major, primal_step, dual_step, halpern)) return rc;
+        if (int rc = launch_iteration(st, P, src, tgt, P.dual[at], P.dual[at ^ 1], checkpoint, major, primal_step, dual_step,
+                                      halpern))
+            return rc;
+        at ^= 1;
         prof_end(st);
         HM_LAUNCH_CHECK("pdhg iteration");
         if (checkpoint) {
