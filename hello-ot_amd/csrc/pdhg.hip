@@ -13,7 +13,7 @@
 //   target order (slot k): edges sorted by target, ascending caller edge id within a target, so target t owns
 //     [off[n+t]-e, off[n+t+1]-e). Arrays: row_t, cs_t, x_t, ax_t, px_t.
 // Both copies receive identical operands in identical order and therefore stay bit-identical.
-// Per node (sources then targets): scale, bs, ns, y, ay, py, dy, and dual = y / ns in two buffers: an iteration reads
+// Per node (sources then targets): scale, bs, ns, y, ay, py, dy, and dual = y / ns in several buffers: an iteration reads
 // the duals of one and writes the next ones to the other.
 //
 // One iteration is one launch: the restatement's two loops (source nodes, then target nodes) both start from the duals
@@ -27,7 +27,8 @@
 // (lanes sum in edge order through shuffles) when every node fits in one chunk of the group, else node blocks
 // (edge-parallel steps, then one thread per node sums its reflections in edge order from LDS). Both are
 // bit-identical to a sequential sum.
-// The only gathers are of duals. Scalars read back to the host only at evaluations and checkpoints.
+// The only gathers are of duals. Scalars read back to the host only at evaluations and checkpoints. Between them, a
+// problem that fits the chip runs its iterations in one launch (see "resident runs").
 //
 // Node numbering: on large problems (at least HELLOOT_PDHG_REORDER nodes, default 2^20, where the duals outgrow
 // an XCD's L2) the nodes are renumbered inside the solve so that nodes joined by many edges get nearby numbers:
@@ -51,6 +52,8 @@ namespace {
 
 constexpr int RB = 1024;     // blocks of the fixed-shape reductions
 constexpr int RT = 256;      // threads per reduction block
+constexpr int RESIDENT_T = 256;        // threads per workgroup of a resident run of iterations
+constexpr int RESIDENT_BLOCKS = 1024;  // its most workgroups
 
 struct Pdhg {
     int64_t n, nt, nodes, e;
@@ -70,7 +73,7 @@ struct Pdhg {
     int32_t *gbase_s, *gbase_t;
     // nodes
     double *scale, *bs, *ns, *y, *ay, *py, *dy;
-    double* dual[2];
+    double* dual[3];
     int32_t *deg, *off, *eid;
     // node numbering (map_s / map_t: internal number of a caller source / target, or null for the identity;
     // inv: caller node of an internal node, sources then targets) and its scratch
@@ -88,6 +91,7 @@ struct Pdhg {
     double* partial;   // RB * 4
     double* result;    // 4
     int* flag;         // 1
+    int32_t* part;     // resident runs: first node of each workgroup
 };
 
 template <class A>
@@ -130,7 +134,9 @@ void pdhg_layout(A& a, int64_t n, int64_t nt, int64_t e, size_t sort_tmp, size_t
     P.sort_tmp = a.template take<char>(sort_tmp > 0 ? sort_tmp : 1);
     P.sort_tmp_bytes = sort_tmp;
     P.partial = a.template take<double>((size_t)RB * 4);
-    P.result = a.template take<double>(4);
+    P.result = a.template take<double>(5);
+    P.part = a.template take<int32_t>(RESIDENT_BLOCKS + 2);
+    P.dual[2] = a.template take<double>(nodes <= (int64_t)RESIDENT_BLOCKS * RESIDENT_T ? nodes : 1);
     P.flag = a.template take<int>(4);
     P.map_s = a.template take<int32_t>(n);
     P.map_t = a.template take<int32_t>(nt);
@@ -712,6 +718,233 @@ __global__ __launch_bounds__(PT) void k_iteration(const Pdhg P, SidePlan src, Si
     }
 }
 
+// ---------------------------------------------------------------------------------------------------------
+// resident runs of iterations
+// ---------------------------------------------------------------------------------------------------------
+// Up to some 2 million edges and nodes the whole iteration state fits the chip's registers, and an iteration of separate
+// launches is bound by latency: the launch, then offsets, edges, gathered duals, each from memory. A resident run does
+// the plain iterations between two checkpoints in one cooperative launch: each workgroup keeps the edges of a run of
+// consecutive nodes of one side in registers (iterate, anchor, cost, gathered node) and its nodes' duals in LDS, and
+// only the duals that other workgroups gather pass through memory.
+//
+// There is no grid barrier: a dual is its own signal. Iteration s reads slot s % 3 of the three dual buffers and
+// publishes to slot (s + 1) % 3; a slot holds UNPUBLISHED until its node's dual arrives, and a reader repeats its load
+// until it sees another value. Every edge is held by both of its ends, so once a workgroup has gathered the duals of
+// iteration s, each node it reads has used this workgroup's duals of iteration s - 1: the workgroup then sets them to
+// UNPUBLISHED again, waits until that store has reached memory, and publishes. A reader that has seen the new dual can
+// therefore only find UNPUBLISHED or a newer dual in the slot it reads next. All loads and stores of duals inside a
+// run have agent scope (they bypass the caches of the XCDs). All workgroups are on the chip at once (the launch is
+// cooperative), and a wait that lasts RESIDENT_WAIT ends the run with an error.
+//
+// Measured, us per iteration, separate launches -> resident: 700 nodes a side and 6 thousand edges 5.2 -> 2.2, 4096 and
+// 61 thousand 8.7 -> 3.3, 16384 and 246 thousand 11.8 -> 7.8, where the gathers that bypass the caches (some 50 per ns)
+// bound it; a grid barrier instead of the signals took 6 at 4096 nodes, with a release fence that writes back L2 14.
+constexpr long long UNPUBLISHED = 0x7FF85E1DE0000001ll;  // a NaN that no operation returns
+constexpr long long RESIDENT_WAIT = 2000000000ll;         // 20 s of the 100 MHz clock
+
+// part[0..ws]: first source node of each of the ws source workgroups (and n), then part[ws+1..]: the same for the
+// targets. Cut at equal weights of a side's nodes in order, a node weighing its degree + k.
+__global__ void k_partition(const int32_t* __restrict__ off, int64_t n, int64_t nt, int64_t e, int ws, int wt, int k,
+                            int32_t* __restrict__ part) {
+    for (int b = blockIdx.x * blockDim.x + threadIdx.x; b < ws + wt + 2; b += gridDim.x * blockDim.x) {
+        const bool source = b <= ws;
+        const int64_t count = source ? n : nt, w = source ? ws : wt, j = source ? b : b - ws - 1;
+        const int32_t* const o = source ? off : off + n;
+        const int64_t first = source ? 0 : e;
+        const int64_t goal = (e + k * count) * j / w;
+        int64_t lo = 0, hi = count;  // the first node whose weight before it reaches the goal
+        while (lo < hi) {
+            const int64_t mid = (lo + hi) / 2;
+            if ((int64_t)o[mid] - first + k * mid >= goal) hi = mid;
+            else lo = mid + 1;
+        }
+        part[b] = (int32_t)(j == w ? count : lo);
+    }
+}
+
+// no dual published yet in the two buffers that a resident run writes first
+__global__ void k_unpublish(double* __restrict__ a, double* __restrict__ b, int64_t nodes) {
+    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < nodes; i += (int64_t)gridDim.x * blockDim.x) {
+        a[i] = __longlong_as_double(UNPUBLISHED);
+        b[i] = __longlong_as_double(UNPUBLISHED);
+    }
+}
+
+__device__ __forceinline__ bool unpublished(double v) { return __double_as_longlong(v) == UNPUBLISHED; }
+
+// `steps` iterations, none of them a checkpoint, from the duals in `cur`; the last ones end up in the buffer that `steps`
+// rotations of (cur, next, spare) bring to the front. Workgroups [0, ws) hold source nodes, the rest target nodes:
+// at most RESIDENT_T * K edges and RESIDENT_T nodes each. Same operations, operands and order as k_iteration.
+// K = 8 leaves 128 registers a thread (four workgroups on a CU), which it fills.
+template <int K>
+__global__ __launch_bounds__(RESIDENT_T, K > 4 ? 4 : 1) void k_resident(const Pdhg P, int ws, int steps, int64_t inner,
+                                                                      double* cur, double* next, double* spare,
+                                                                      double primal_step, double dual_step) {
+    constexpr int T = RESIDENT_T;
+    __shared__ double refl[T * K];
+    __shared__ double dual[T];
+    __shared__ int late;
+    const int tid = threadIdx.x;
+    const bool source = (int)blockIdx.x < ws;
+    const int b = source ? blockIdx.x : blockIdx.x + 1;
+    const int32_t p0 = P.part[b], p1 = P.part[b + 1];
+    const int64_t first = (source ? 0 : P.n) + p0;
+    const int nn = p1 - p0;
+    const int32_t ebase = source ? 0 : (int32_t)P.e;
+    const int32_t e0 = P.off[first] - ebase;
+    const int len = P.off[first + nn] - ebase - e0;
+    double* const xs = (source ? P.x : P.x_t) + e0;
+    const double* const axs = (source ? P.ax : P.ax_t) + e0;
+    const double* const css = (source ? P.cs : P.cs_t) + e0;
+    const int32_t* const own = (source ? P.row : P.col_t) + e0;
+    const int32_t* const far = (source ? P.col : P.row_t) + e0;
+    const int32_t other = source ? (int32_t)P.n : 0;
+    double x[K], ax[K], cs[K];
+    int32_t gi[K], loc[K];
+#pragma unroll
+    for (int u = 0; u < K; ++u) {
+        const int q = u * T + tid;
+        const bool in = q < len;
+        x[u] = in ? xs[q] : 0.0;
+        ax[u] = in ? axs[q] : 0.0;
+        cs[u] = in ? css[q] : 0.0;
+        loc[u] = in ? own[q] - p0 : 0;
+        gi[u] = in ? other + far[q] : 0;
+    }
+    double y = 0.0, ns = 1.0, bs = 0.0, ay = 0.0;
+    int k0 = 0, k1 = 0;
+    if (tid < nn) {
+        const int64_t i = first + tid;
+        y = P.y[i];
+        ns = P.ns[i];
+        bs = P.bs[i];
+        ay = P.ay[i];
+        dual[tid] = cur[i];
+        k0 = P.off[i] - ebase - e0;
+        k1 = P.off[i + 1] - ebase - e0;
+    }
+    if (tid == 0) late = 0;
+    __syncthreads();
+    for (int s = 0; s < steps; ++s) {
+        double g[K];
+#pragma unroll
+        for (int u = 0; u < K; ++u) {
+            g[u] = 0.0;
+            if (u * T + tid < len) g[u] = __hip_atomic_load(cur + gi[u], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        const double halpern = double(inner + s + 1) / double(inner + s + 2);
+        const double keep = 1.0 - halpern;
+        if (s > 0) {
+            bool miss = false;
+#pragma unroll
+            for (int u = 0; u < K; ++u) miss |= unpublished(g[u]);
+            if (__any(miss)) {
+                const long long from = wall_clock64();
+                do {
+                    miss = false;
+#pragma unroll
+                    for (int u = 0; u < K; ++u)
+                        if (unpublished(g[u]))
+                            g[u] = __hip_atomic_load(cur + gi[u], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+                    for (int u = 0; u < K; ++u) miss |= unpublished(g[u]);
+                    if (wall_clock64() - from > RESIDENT_WAIT) {
+                        late = 1;
+                        break;
+                    }
+                } while (__any(miss));
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < K; ++u) {
+            const double at = dual[loc[u]] + g[u];
+            const double pxj = fmax(x[u] - primal_step * (cs[u] - at), 0.0);
+            const double r = 2.0 * pxj - x[u];
+            x[u] = halpern * r + keep * ax[u];
+            refl[u * T + tid] = r;
+        }
+        __syncthreads();
+        if (late) {
+            if (tid == 0) P.result[4] = 1.0;
+            return;
+        }
+        if (tid < nn) {
+            __hip_atomic_store(spare + first + tid, __longlong_as_double(UNPUBLISHED), __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
+            const double sum = fold_in_order(refl, k0, k1, 0.0);
+            const double py = y - dual_step * (sum / ns - bs);
+            const double r = 2.0 * py - y;
+            y = halpern * r + keep * ay;
+            const double d = y / ns;
+            dual[tid] = d;
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            __hip_atomic_store(next + first + tid, unpublished(d) ? __builtin_nan("") : d, __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
+        }
+        __syncthreads();
+        double* const t = cur;
+        cur = next;
+        next = spare;
+        spare = t;
+    }
+#pragma unroll
+    for (int u = 0; u < K; ++u)
+        if (u * T + tid < len) xs[u * T + tid] = x[u];
+    if (tid < nn) P.y[first + tid] = y;
+}
+
+struct ResidentPlan {
+    int k, ws, wt;  // edges per thread (0: separate launches), workgroups of the two sides
+};
+
+// Fewest workgroups that surely hold a side. k_partition cuts at equal weights, a node weighing its degree + k, so a
+// workgroup's weight stays below its share + the heaviest node; at most RESIDENT_T * k of weight means at most
+// RESIDENT_T * k edges and RESIDENT_T nodes.
+inline int64_t resident_blocks(int64_t e, int64_t nodes, int max_degree, int k) {
+    const int64_t room = (int64_t)RESIDENT_T * k - max_degree - k - 1;
+    return room < 1 ? INT32_MAX : (e + k * nodes + room - 1) / room;
+}
+
+inline const void* resident_kernel(int k) {
+    return k == 2   ? reinterpret_cast<const void*>(k_resident<2>)
+           : k == 4 ? reinterpret_cast<const void*>(k_resident<4>)
+                    : reinterpret_cast<const void*>(k_resident<8>);
+}
+
+// Edges per thread: the fewest that need no more than a workgroup per CU (a second one on the CU shares its gather
+// path: at 4096 nodes a side 213 workgroups of 4 edges a thread take 3.3 us an iteration, 433 of 2 take 4.5, 118 of 8
+// take 3.8), else 8 if all fit on the chip at once. Larger problems keep the separate launches, whose gathers hit L2:
+// the two are level where the chip is full.
+inline ResidentPlan resident_plan(int64_t n, int64_t nt, int64_t e, int max_s, int max_t) {
+    int device = 0, cus = 0, cooperative = 0, per_cu = 0;
+    if (hipGetDevice(&device) != hipSuccess ||
+        hipDeviceGetAttribute(&cooperative, hipDeviceAttributeCooperativeLaunch, device) != hipSuccess || !cooperative ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess)
+        return {0, 0, 0};
+    for (int k = 2; k <= 8; k *= 2) {
+        const int64_t ws = resident_blocks(e, n, max_s, k), wt = resident_blocks(e, nt, max_t, k);
+        if (ws + wt > (k < 8 ? cus : RESIDENT_BLOCKS)) continue;
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, resident_kernel(k), RESIDENT_T, 0) != hipSuccess) break;
+        if (ws + wt <= (int64_t)per_cu * cus) return {k, (int)ws, (int)wt};
+    }
+    return {0, 0, 0};
+}
+
+// shortest run worth its two launches and the load and store of the state (some 30 us; an iteration saves 3 to 5)
+constexpr int64_t RESIDENT_STEPS = 16;
+constexpr int64_t RESIDENT_MOST = 4096;  // keeps a launch under some 50 ms
+
+int launch_resident(hipStream_t st, const Pdhg& P, const ResidentPlan& rp, int steps, int64_t inner, double* cur,
+                    double* next, double* spare, double ps, double ds) {
+    hipLaunchKernelGGL(k_unpublish, dim3(64), dim3(256), 0, st, next, spare, P.nodes);
+    HM_LAUNCH_CHECK("k_unpublish");
+    Pdhg p = P;
+    int ws = rp.ws;
+    void* args[] = {&p, &ws, &steps, &inner, &cur, &next, &spare, &ps, &ds};
+    HM_HIP(hipLaunchCooperativeKernel(resident_kernel(rp.k), dim3(rp.ws + rp.wt), dim3(RESIDENT_T), args, 0, st));
+    return HM_OK;
+}
+
 __global__ void k_restart(const Pdhg P, double* __restrict__ dual) {
     const int64_t total = P.e > P.nodes ? P.e : P.nodes;
     for (int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; j < total; j += (int64_t)gridDim.x * blockDim.x) {
@@ -822,8 +1055,9 @@ int number_nodes(hipStream_t st, const int64_t* rows, const int64_t* cols, int64
 int read_result(hipStream_t st, const Pdhg& P, int q, double* host) {
     hipLaunchKernelGGL(k_combine, dim3(1), dim3(RT), 0, st, P.partial, P.result, q);
     HM_LAUNCH_CHECK("k_combine");
-    HM_HIP(hipMemcpyAsync(host, P.result, sizeof(double) * q, hipMemcpyDeviceToHost, st));
+    HM_HIP(hipMemcpyAsync(host, P.result, sizeof(double) * 5, hipMemcpyDeviceToHost, st));
     HM_HIP(hipStreamSynchronize(st));
+    if (host[4] != 0.0) return fail(HM_EHIP, "PDHG: a workgroup of a resident run did not answer in time");
     return HM_OK;
 }
 
@@ -871,6 +1105,7 @@ extern "C" int hm_pdhg_solve(void* stream, const int64_t* rows, const int64_t* c
     // ---- LP assembly: node numbers, endpoints, degrees, per-node incident edge lists (ascending edge id) ----
     hipLaunchKernelGGL(k_fill_i32, dim3(grid_of(nodes + 1)), dim3(256), 0, st, P.deg, nodes + 1, 0);
     hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, st, P.flag, 4, 0);
+    hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, st, reinterpret_cast<int32_t*>(P.result + 4), 2, 0);
     if (nodes >= reorder_min_nodes()) {
         if (int rc = number_nodes(st, rows, cols, n, nt, e, P)) return rc;
     } else {
@@ -892,7 +1127,7 @@ extern "C" int hm_pdhg_solve(void* stream, const int64_t* rows, const int64_t* c
                                               (int)(2 * e), 0, end_bit_for(nodes), st));
 
     // ---- scaling (solver.cpp:91-110) ----
-    double host[4];
+    double host[5];
     hipLaunchKernelGGL(k_sumsq, dim3(RB), dim3(RT), 0, st, masses, nodes, P.partial);
     HM_LAUNCH_CHECK("k_sumsq");
     if (int rc = read_result(st, P, 1, host)) return rc;
@@ -950,6 +1185,12 @@ extern "C" int hm_pdhg_solve(void* stream, const int64_t* rows, const int64_t* c
                            nt, tgt.npb, (int32_t)e, P.row_t, P.gbase_t, P.g16_t);
     }
     HM_LAUNCH_CHECK("node-block setup");
+    const ResidentPlan resident = resident_plan(n, nt, e, flag[1], flag[2]);
+    if (resident.k > 0) {
+        hipLaunchKernelGGL(k_partition, dim3(1), dim3(256), 0, st, P.off, n, nt, e, resident.ws, resident.wt, resident.k,
+                           P.part);
+        HM_LAUNCH_CHECK("k_partition");
+    }
     for (;;) {
         if (local_count % freq == 0) {
             hipLaunchKernelGGL(k_evaluate, dim3(RB), dim3(RT), 0, st, P, masses, costs, variable, bound, objective,
@@ -1016,10 +1257,23 @@ extern "C" int hm_pdhg_solve(void* stream, const int64_t* rows, const int64_t* c
         const bool checkpoint = major || is_restart;
         // px / py are read only by the evaluation that follows a major iteration
         prof_begin(st, "pdhg_iteration");
-        if (int rc = launch_iteration(st, P, src, tgt, P.dual[at], P.dual[at ^ 1], checkpoint, major, primal_step, dual_step,
+        const int64_t plain = freq - 1 - local_count % freq;  // iterations before the next major one
+        const int64_t steps = plain < RESIDENT_MOST ? plain : RESIDENT_MOST;
+        if (resident.k > 0 && !checkpoint && steps >= RESIDENT_STEPS) {
+            if (int rc = launch_resident(st, P, resident, (int)steps, local_inner, P.dual[at], P.dual[(at + 1) % 3],
+                                         P.dual[(at + 2) % 3], primal_step, dual_step))
+                return rc;
+            prof_end(st);
+            prof_count("pdhg_iteration", steps - 1);
+            at = (int)((at + steps) % 3);
+            local_count += steps;
+            local_inner += steps;
+            continue;
+        }
+        if (int rc = launch_iteration(st, P, src, tgt, P.dual[at], P.dual[at == 0], checkpoint, major, primal_step, dual_step,
                                       halpern))
             return rc;
-        at ^= 1;
+        at = at == 0;
         prof_end(st);
         HM_LAUNCH_CHECK("pdhg iteration");
         if (checkpoint) {

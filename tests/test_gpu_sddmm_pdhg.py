@@ -375,6 +375,50 @@ def test_pdhg_with_internal_node_numbers_matches_oracle(cuda, monkeypatch, name)
     assert out["1"].obj_val == pytest.approx(out["off"].obj_val, rel=1e-12)
 
 
+@pytest.mark.parametrize("ns,nt,per_row,hub,freq,checks", [
+    (2, 3, 3, 0, 17, 3),          # the smallest: one workgroup a side, runs of exactly 16 iterations
+    (700, 300, 5, 0, 40, 3),      # 2 edges a thread, degrees of the two sides apart
+    (700, 700, 5, 490, 16, 3),    # runs of 15: separate launches
+    (700, 700, 5, 490, 40, 2),    # a hub that all but fills a workgroup of 2 edges a thread
+    (700, 700, 5, 600, 40, 2),    # one that needs 4
+    (3000, 2500, 4, 2030, 40, 2),  # one that all but fills a workgroup of 8
+    (3000, 2500, 4, 2045, 40, 2),  # one that no workgroup holds: separate launches
+    (4096, 4096, 12, 0, 40, 2),   # 4 edges a thread
+    (16384, 12000, 10, 30, 40, 2),  # 8 edges a thread, more than a workgroup per CU
+    (300, 300, 2, 0, 4200, 1),    # more iterations than one launch runs
+])
+def test_pdhg_resident_runs_match_oracle(cuda, ns, nt, per_row, hub, freq, checks):
+    """The iterations between checkpoints in one cooperative launch, over its shapes and the edges of their rules. The
+    last source and target have no edges where a side has more than 200 nodes; edge lists in random order; warm start."""
+    rng = np.random.default_rng(ns + hub + freq)
+    live_s, live_t = ns - (ns > 200), nt - (nt > 200)
+    cols = [rng.choice(live_t, min(per_row, live_t), replace=False) for _ in range(live_s)]
+    rows = np.repeat(np.arange(live_s), min(per_row, live_t))
+    extra = np.setdiff1d(np.arange(hub), rows[np.concatenate(cols) == 0]) if hub else np.empty(0, np.int64)
+    rows = np.concatenate((rows, extra))
+    cols = np.concatenate(cols + [np.zeros(extra.size, np.int64)])
+    missing = np.setdiff1d(np.arange(live_t), cols)
+    rows = np.concatenate((rows, rng.integers(0, live_s, missing.size)))
+    cols = np.concatenate((cols, missing))
+    perm = rng.permutation(rows.size)
+    rows, cols = rows[perm].astype(np.int64), cols[perm].astype(np.int64)
+    costs = rng.random(rows.size)
+    a, b = np.zeros(ns), np.zeros(nt)
+    a[:live_s], b[:live_t] = rng.random(live_s), rng.random(live_t)
+    a /= a.sum()
+    b /= b.sum()
+    x0, y0 = rng.random(rows.size) / rows.size, 0.1 * rng.standard_normal(ns + nt)
+    ref = oracle.pdhg_solve(rows, cols, costs, a, b, warm_start_primal=x0, warm_start_dual=y0,
+                            evaluation_frequency=freq, iteration_limit=freq * checks, tolerance=0.0)
+    r = NativeRestrictedOTPDLP(device=cuda, evaluation_frequency=freq, iteration_limit=freq * checks).solve_restricted(
+        rows=rows, cols=cols, costs=costs, source_mass=a, target_mass=b, tolerance=0.0, warm_start_primal=x0,
+        warm_start_dual=y0)
+    assert r.iterations == ref["iterations"] == freq * checks
+    assert r.solver_diag["restart_count"] == ref["restart_count"]
+    np.testing.assert_allclose(r.x.cpu().numpy(), ref["x"], rtol=1e-9, atol=1e-12)
+    np.testing.assert_allclose(r.y.cpu().numpy(), ref["y"], rtol=1e-9, atol=1e-12)
+
+
 def test_pdhg_internal_numbering_validates_endpoints(cuda, monkeypatch):
     """The library's own check (the Python wrapper validates first), on the numbering path."""
     from hello_ot_amd.lp.native_pdlp import run_pdhg
