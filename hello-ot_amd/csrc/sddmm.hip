@@ -11,6 +11,84 @@
 namespace hm {
 namespace {
 
+// Pair costs gather a row (or two) per pair: what bounds them is how much of a row a wave asks for at a time.
+// Rows that are 16-byte aligned (d a multiple of 4) are read 16 bytes at a time: 16 lanes per pair, a wave four pairs,
+// lane t of the 16 accumulating features 4 t .. 4 t + 3 of every 64. quad_tree finishes the fixed order: its four
+// accumulators are lanes 4 t .. 4 t + 3 of the 64, so strides 32 to 4 are lane strides 8 to 1 and the last two lie
+// within a lane. 1.5 million pairs of 2048 features, 12.3 GB of gathered rows: 3.25 -> 1.8 ms (6.8 TB/s, the rate of the
+// last-level cache); as 64 lanes of 4 bytes each wave had one pair's rows in flight.
+__device__ __forceinline__ double quad_tree_sum(double (&a)[4]) {
+#pragma unroll
+    for (int s = 8; s >= 1; s >>= 1)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) a[c] = a[c] + __shfl_down(a[c], s, 16);
+    a[0] = a[0] + a[2];
+    a[1] = a[1] + a[3];
+    return a[0] + a[1];
+}
+__device__ __forceinline__ double quad_tree_max(double (&a)[4]) {
+#pragma unroll
+    for (int s = 8; s >= 1; s >>= 1)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) a[c] = fmax(a[c], __shfl_down(a[c], s, 16));
+    return fmax(fmax(a[0], a[2]), fmax(a[1], a[3]));
+}
+
+// the products are exact in fp64, so the fused form rounds like a multiply and an add
+__device__ __forceinline__ void quad_fma(double (&a)[4], const float4 x, const float4 y) {
+    a[0] = fma((double)x.x, (double)y.x, a[0]);
+    a[1] = fma((double)x.y, (double)y.y, a[1]);
+    a[2] = fma((double)x.z, (double)y.z, a[2]);
+    a[3] = fma((double)x.w, (double)y.w, a[3]);
+}
+
+inline bool quad_rows(const float* X, const float* Y, int d) {
+    return d % 4 == 0 && ((reinterpret_cast<uintptr_t>(X) | reinterpret_cast<uintptr_t>(Y)) & 15) == 0;
+}
+
+__device__ __forceinline__ double quad_dot64(const float* __restrict__ x, const float* __restrict__ y, int d, int t) {
+    double a[4] = {0.0, 0.0, 0.0, 0.0};
+    for (int k = 4 * t; k < d; k += 64)
+        quad_fma(a, *reinterpret_cast<const float4*>(x + k), *reinterpret_cast<const float4*>(y + k));
+    return quad_tree_sum(a);
+}
+
+// CSR rows: one wave per row, four entries at a time
+__global__ __launch_bounds__(256) void sddmm_quad_kernel(const float* __restrict__ X, const float* __restrict__ Y,
+                                                         const double* __restrict__ p, const double* __restrict__ q,
+                                                         const int32_t* __restrict__ rowptr,
+                                                         const int32_t* __restrict__ col, int64_t m, int d,
+                                                         double scale, double* __restrict__ out) {
+    const int lane = threadIdx.x & 63, t = lane & 15, g = lane >> 4;
+    const int64_t waves = (int64_t)gridDim.x * (blockDim.x >> 6);
+    for (int64_t row = (int64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6); row < m; row += waves) {
+        const int32_t e1 = rowptr[row + 1];
+        int32_t e = rowptr[row] + g;
+        int32_t next = e < e1 ? col[e] : 0;
+        for (; e < e1; e += 4) {
+            const int64_t j = next;
+            if (e + 4 < e1) next = col[e + 4];
+            const double dot = quad_dot64(X + row * (int64_t)d, Y + j * (int64_t)d, d, t);
+            if (t == 0) out[e] = (p[row] + q[j]) - scale * dot;
+        }
+    }
+}
+
+// COO pairs
+__global__ __launch_bounds__(256) void pair_costs_quad_kernel(const float* __restrict__ X, const float* __restrict__ Y,
+                                                              const double* __restrict__ p, const double* __restrict__ q,
+                                                              const int64_t* __restrict__ rows,
+                                                              const int64_t* __restrict__ cols, int64_t count, int d,
+                                                              double scale, double* __restrict__ out) {
+    const int t = threadIdx.x & 15;
+    const int64_t quads = (int64_t)gridDim.x * 16;
+    for (int64_t e = (int64_t)blockIdx.x * 16 + (threadIdx.x >> 4); e < count; e += quads) {
+        const int64_t i = rows[e], j = cols[e];
+        const double dot = quad_dot64(X + i * d, Y + j * d, d, t);
+        if (t == 0) out[e] = (p[i] + q[j]) - scale * dot;
+    }
+}
+
 // CSR rows: one wave per row, x_i cached in registers when d <= 64*XR.
 template <int XR>
 __global__ __launch_bounds__(256) void sddmm_l2sq_csr_kernel(const float* __restrict__ X, const float* __restrict__ Y,
@@ -114,6 +192,35 @@ __global__ __launch_bounds__(256) void pair_costs_l2sq_kernel(const float* __res
     }
 }
 
+template <int KIND>
+__device__ __forceinline__ double norm_term(double a, float x, float y) {
+    const double z = (double)x - (double)y;
+    return KIND == HM_COST_L1 ? a + fabs(z) : KIND == HM_COST_LINF ? fmax(a, fabs(z)) : a + z * z;
+}
+
+template <int KIND>
+__global__ __launch_bounds__(256) void pair_costs_norm_quad_kernel(const float* __restrict__ X, const float* __restrict__ Y,
+                                                                   const int64_t* __restrict__ rows,
+                                                                   const int64_t* __restrict__ cols, int64_t count, int d,
+                                                                   double* __restrict__ out) {
+    const int t = threadIdx.x & 15;
+    const int64_t quads = (int64_t)gridDim.x * 16;
+    for (int64_t e = (int64_t)blockIdx.x * 16 + (threadIdx.x >> 4); e < count; e += quads) {
+        const float* x = X + rows[e] * d;
+        const float* y = Y + cols[e] * d;
+        double a[4] = {0.0, 0.0, 0.0, 0.0};
+        for (int k = 4 * t; k < d; k += 64) {
+            const float4 u = *reinterpret_cast<const float4*>(x + k), v = *reinterpret_cast<const float4*>(y + k);
+            a[0] = norm_term<KIND>(a[0], u.x, v.x);
+            a[1] = norm_term<KIND>(a[1], u.y, v.y);
+            a[2] = norm_term<KIND>(a[2], u.z, v.z);
+            a[3] = norm_term<KIND>(a[3], u.w, v.w);
+        }
+        const double r = (KIND == HM_COST_LINF) ? quad_tree_max(a) : quad_tree_sum(a);
+        if (t == 0) out[e] = (KIND == HM_COST_L2) ? sqrt(r) : r;
+    }
+}
+
 template <int G, int KIND>
 __global__ __launch_bounds__(256) void pair_costs_norm_kernel(const float* __restrict__ X, const float* __restrict__ Y,
                                                               const int64_t* __restrict__ rows,
@@ -137,28 +244,45 @@ __global__ __launch_bounds__(256) void pair_costs_norm_kernel(const float* __res
 }
 
 // fp32 norm costs exactly as the pricing scan forms them: 32-feature chunks accumulated sequentially in fp32,
-// chunk results combined in order, l2 = sqrt in fp64 of the fp32 sum, rounded once to fp32.
-template <int KIND>
+// chunk results combined in order, l2 = sqrt in fp64 of the fp32 sum, rounded once to fp32. G lanes per pair, one chunk
+// each: the lanes read the rows side by side and each then adds the chunk results in their order.
+template <int KIND, int G, bool WIDE>
 __global__ __launch_bounds__(256) void pair_costs_norm32_kernel(const float* __restrict__ X, const float* __restrict__ Y,
                                                                 const int64_t* __restrict__ rows,
                                                                 const int64_t* __restrict__ cols, int64_t count, int d,
                                                                 double* __restrict__ out) {
-    for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < count; e += (int64_t)gridDim.x * blockDim.x) {
+    const int g = threadIdx.x % G;
+    const int64_t groups = (int64_t)gridDim.x * (256 / G);
+    auto term = [](float part, float a, float b) {
+        const float z = a - b;
+        return KIND == HM_COST_L1 ? part + fabsf(z) : KIND == HM_COST_LINF ? fmaxf(part, fabsf(z)) : fmaf(z, z, part);
+    };
+    for (int64_t e = (int64_t)blockIdx.x * (256 / G) + threadIdx.x / G; e < count; e += groups) {
         const float* x = X + rows[e] * d;
         const float* y = Y + cols[e] * d;
         float acc = 0.0f;
-        for (int base = 0; base < d; base += 32) {
-            float part = 0.0f;
+        for (int first = 0; first < d; first += 32 * G) {
+            const int base = first + 32 * g;
             const int end = base + 32 < d ? base + 32 : d;
-            for (int k = base; k < end; ++k) {
-                const float z = x[k] - y[k];
-                if (KIND == HM_COST_L1) part = part + fabsf(z);
-                else if (KIND == HM_COST_LINF) part = fmaxf(part, fabsf(z));
-                else part = fmaf(z, z, part);
+            float part = 0.0f;
+            if (WIDE) {
+                for (int k = base; k < end; k += 4) {
+                    const float4 u = *reinterpret_cast<const float4*>(x + k), v = *reinterpret_cast<const float4*>(y + k);
+                    part = term(part, u.x, v.x);
+                    part = term(part, u.y, v.y);
+                    part = term(part, u.z, v.z);
+                    part = term(part, u.w, v.w);
+                }
+            } else {
+                for (int k = base; k < end; ++k) part = term(part, x[k], y[k]);
             }
-            acc = (KIND == HM_COST_LINF) ? fmaxf(acc, part) : acc + part;
+#pragma unroll
+            for (int c = 0; c < G; ++c) {
+                const float other = G == 1 ? part : __shfl(part, c, G);
+                if (first + 32 * c < d) acc = (KIND == HM_COST_LINF) ? fmaxf(acc, other) : acc + other;
+            }
         }
-        out[e] = (KIND == HM_COST_L2) ? (double)(float)sqrt((double)acc) : (double)acc;
+        if (g == 0) out[e] = (KIND == HM_COST_L2) ? (double)(float)sqrt((double)acc) : (double)acc;
     }
 }
 
@@ -188,7 +312,12 @@ extern "C" int hm_sddmm_l2sq_csr(void* stream, const float* X, const float* Y, c
 #define HM_SDDMM(XR) \
     hipLaunchKernelGGL((sddmm_l2sq_csr_kernel<XR>), dim3(grid), dim3(256), 0, st, X, Y, p, q, rowptr, col, m, d, scale, out)
     prof_begin(st, "sddmm_l2sq_csr");
-    if (d <= 64) HM_SDDMM(1);
+    // level between 128 and 256 features (262144 rows of 16 entries, d = 256: 0.74 ms and 0.75 in fours, 5.7 TB/s of
+    // gathered rows); elsewhere the fours are ahead (30000 rows of 20, d = 1024: 0.69 -> 0.41 ms; 60000 rows of 20,
+    // d = 128: 0.19 -> 0.12)
+    if (quad_rows(X, Y, d) && (d <= 128 || d > 256))
+        hipLaunchKernelGGL(sddmm_quad_kernel, dim3(grid), dim3(256), 0, st, X, Y, p, q, rowptr, col, m, d, scale, out);
+    else if (d <= 64) HM_SDDMM(1);
     else if (d <= 128) HM_SDDMM(2);
     else if (d <= 256) HM_SDDMM(4);
     else if (d <= 512) HM_SDDMM(8);
@@ -211,7 +340,11 @@ extern "C" int hm_pair_costs_l2sq(void* stream, const float* X, const float* Y, 
 #define HM_PAIRS(GG)                                                                                            \
     hipLaunchKernelGGL((pair_costs_l2sq_kernel<GG>), dim3(grid_for(count, 256 / GG)), dim3(256), 0, st, X, Y, p, q, \
                        rows, cols, count, d, scale, out)
-    if (G == 8) HM_PAIRS(8);
+    // (up to 16 features the groups below use more of their lanes)
+    if (d > 16 && quad_rows(X, Y, d))
+        hipLaunchKernelGGL(pair_costs_quad_kernel, dim3(grid_for(count, 16)), dim3(256), 0, st, X, Y, p, q, rows, cols,
+                           count, d, scale, out);
+    else if (G == 8) HM_PAIRS(8);
     else if (G == 16) HM_PAIRS(16);
     else if (G == 32) HM_PAIRS(32);
     else HM_PAIRS(64);
@@ -237,7 +370,15 @@ extern "C" int hm_pair_costs_norm(void* stream, const float* X, const float* Y, 
         else if (kind == HM_COST_LINF) HM_NORM(GG, HM_COST_LINF); \
         else HM_NORM(GG, HM_COST_L2);                        \
     } while (0)
-    if (G == 8) HM_NORM_K(8);
+    if (d > 16 && quad_rows(X, Y, d)) {
+#define HM_NORM_QUAD(KK)                                                                                               \
+    hipLaunchKernelGGL((pair_costs_norm_quad_kernel<KK>), dim3(grid_for(count, 16)), dim3(256), 0, st, X, Y, rows, cols, \
+                       count, d, out)
+        if (kind == HM_COST_L1) HM_NORM_QUAD(HM_COST_L1);
+        else if (kind == HM_COST_LINF) HM_NORM_QUAD(HM_COST_LINF);
+        else HM_NORM_QUAD(HM_COST_L2);
+#undef HM_NORM_QUAD
+    } else if (G == 8) HM_NORM_K(8);
     else if (G == 16) HM_NORM_K(16);
     else if (G == 32) HM_NORM_K(32);
     else HM_NORM_K(64);
@@ -254,16 +395,29 @@ extern "C" int hm_pair_costs_norm_fp32(void* stream, const float* X, const float
     if (count == 0) return HM_OK;
     HM_CHECK_ARG(X && Y && rows && cols && out, "pair costs: null pointer argument");
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-    const unsigned grid = grid_for(count, 256);
-    if (kind == HM_COST_L1)
-        hipLaunchKernelGGL((pair_costs_norm32_kernel<HM_COST_L1>), dim3(grid), dim3(256), 0, st, X, Y, rows, cols, count, d,
-                           out);
-    else if (kind == HM_COST_LINF)
-        hipLaunchKernelGGL((pair_costs_norm32_kernel<HM_COST_LINF>), dim3(grid), dim3(256), 0, st, X, Y, rows, cols, count,
-                           d, out);
-    else
-        hipLaunchKernelGGL((pair_costs_norm32_kernel<HM_COST_L2>), dim3(grid), dim3(256), 0, st, X, Y, rows, cols, count, d,
-                           out);
+    const bool wide = quad_rows(X, Y, d);
+#define HM_NORM32(KK, GG)                                                                                            \
+    do {                                                                                                             \
+        if (wide)                                                                                                    \
+            hipLaunchKernelGGL((pair_costs_norm32_kernel<KK, GG, true>), dim3(grid_for(count, 256 / GG)), dim3(256), \
+                               0, st, X, Y, rows, cols, count, d, out);                                              \
+        else                                                                                                         \
+            hipLaunchKernelGGL((pair_costs_norm32_kernel<KK, GG, false>), dim3(grid_for(count, 256 / GG)),           \
+                               dim3(256), 0, st, X, Y, rows, cols, count, d, out);                                   \
+    } while (0)
+#define HM_NORM32_K(GG)                                         \
+    do {                                                        \
+        if (kind == HM_COST_L1) HM_NORM32(HM_COST_L1, GG);      \
+        else if (kind == HM_COST_LINF) HM_NORM32(HM_COST_LINF, GG); \
+        else HM_NORM32(HM_COST_L2, GG);                         \
+    } while (0)
+    // a lane per chunk, up to 16 (a thread per pair read rows 4 bytes at a time, a line apart from its neighbours): 200
+    // thousand pairs of 4096 features 12.4 -> 3.5 ms, 2 million of 64 0.71 -> 0.23
+    if (d <= 32) HM_NORM32_K(1);
+    else if (d <= 128) HM_NORM32_K(4);
+    else HM_NORM32_K(16);
+#undef HM_NORM32_K
+#undef HM_NORM32
     HM_LAUNCH_CHECK("pair_costs_norm_fp32");
     return HM_OK;
 }

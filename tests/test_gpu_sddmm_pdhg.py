@@ -93,6 +93,37 @@ def _small_problem():
                 source_mass=np.array([0.4, 0.6]), target_mass=np.array([0.5, 0.5]))
 
 
+@pytest.mark.parametrize("d", [4, 20, 36, 68, 128, 132, 260, 1028])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_pair_costs_of_wide_and_shifted_rows_bit_exact(cuda, d, shift):
+    """Rows read 16 bytes at a time (d a multiple of 4 on an aligned buffer), with features left over beyond 16 lanes,
+    and the same rows from a buffer that starts 4 bytes later (read 4 bytes at a time), against the oracle: the same
+    bits in CSR and pair order, fp64 and fp32 norms."""
+    rng = np.random.default_rng(7 * d)
+    X, Y = rng.random((40, d)).astype(np.float32), rng.random((50, d)).astype(np.float32)
+    p, q = (X.astype(np.float64) ** 2).sum(1), (Y.astype(np.float64) ** 2).sum(1)
+    rows, cols = np.sort(rng.integers(0, 40, 777)), rng.integers(0, 50, 777)
+    rowptr = np.searchsorted(rows, np.arange(41)).astype(np.int32)
+
+    def on(a):
+        flat = torch.empty(a.size + shift, dtype=torch.float32, device=cuda)
+        flat[shift:] = torch.as_tensor(a.ravel()).to(cuda)
+        return flat[shift:].view(a.shape)
+
+    tX, tY = on(X), on(Y)
+    tp, tq, tr, tc = (torch.as_tensor(a).to(cuda) for a in (p, q, rows, cols))
+    ref = oracle.sddmm_l2sq(X, Y, p, q, rowptr, cols.astype(np.int32), 2.0)
+    np.testing.assert_array_equal(lowrank_pair_costs(tX, tY, tp, tq, tr, tc).cpu().numpy(), ref)
+    csr = lowrank_csr_costs(tX, tY, tp, tq, torch.as_tensor(rowptr).to(cuda), tc.int())
+    np.testing.assert_array_equal(csr.cpu().numpy(), ref)
+    for kind in (0, 1, 2):
+        np.testing.assert_array_equal(norm_pair_costs(tX, tY, tr, tc, kind).cpu().numpy(),
+                                      oracle.pair_costs_norm(X, Y, rows, cols, kind))
+        _, cost = oracle.norm_matrices(X, Y, np.zeros(40), np.zeros(50), kind)
+        np.testing.assert_array_equal(norm_pair_costs(tX, tY, tr, tc, kind, precision="fp32").cpu().numpy(),
+                                      cost[rows, cols])
+
+
 @pytest.mark.parametrize("warm", [False, True])
 def test_pdhg_kat_small_problem(cuda, warm):
     # tests/torch_restricted_ot_pdlp_test.py:58-80
