@@ -534,8 +534,9 @@ __device__ __forceinline__ void sweep_row_init(SweepRow<K1>& s, int64_t row, int
 // w = scale*dot + db into the row list (or appends for the wide pass), adds the certificate terms and, with COLS,
 // passes the tile's scores scale*dot + qb through LDS so that each Y row keeps its best K1 over the workgroup's
 // 128 X rows, CPASS Y rows at a time (sC holds CPASS * CST floats; 256 / CPASS threads scan each row and merge
-// their lists). Ends with a barrier: the next tile may rewrite sDB / sGE / sC.
-template <int K1, bool COLS, bool APPEND, int CPASS, bool FULL, bool ST, bool SRT = false>
+// their lists). Ends with a barrier, so that the next tile may rewrite sDB / sGE / sC (SYNC; a sweep that keeps two
+// sets of them and no columns has its own barrier per tile).
+template <int K1, bool COLS, bool APPEND, int CPASS, bool FULL, bool ST, bool SRT = false, bool SYNC = true>
 __device__ __forceinline__ void sweep_epilogue(const v16f (&tot)[NB], SweepRow<K1>& s, int tid, int wave, int h,
                                                int r, int64_t ytile, int64_t y_end, int64_t x0, int64_t panel,
                                                int64_t n, float scale, int STATS_, float slack, const double* sQB64,
@@ -715,7 +716,7 @@ __device__ __forceinline__ void sweep_epilogue(const v16f (&tot)[NB], SweepRow<K
             }
         }
     }
-    __syncthreads();  // all epilogue reads of sDB/sGE/sC finish before the next tile rewrites them
+    if (SYNC) __syncthreads();  // all epilogue reads of sDB/sGE/sC finish before the next tile rewrites them
 }
 
 // End of a sweep workgroup: lane lists -> part[(seg*rows + local row)*2 + h][K1], certificate partials reduced
@@ -964,6 +965,151 @@ __global__ __launch_bounds__(256) void l2sq_sweep(
 #undef HM_EPILOGUE
     }
     sweep_finish<K1, APPEND>(s, tid, lane, wave, h, seg, rows, xb, P, panel, STATS, part, blockstats, sRed);
+}
+
+// fp32 sweep of up to 64 features without column lists: the same products in the same order as l2sq_sweep (steps
+// whose features are all padding left out) and the same epilogue. With so few products per pair the epilogue is most of
+// the work, a chain of LDS reads, compares and votes that one wave per SIMD cannot overlap. The panel's X operands are
+// read once into registers and only Y tiles pass through LDS (two stages, with the tile's biases, one barrier per
+// chunk), so two workgroups fit a CU, and at NC = 1 the products and the epilogue of a tile run without a barrier
+// between them.
+template <int K1, int NC, bool ST>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void l2sq_sweep_short(
+    const float* __restrict__ X, const float* __restrict__ Y, int64_t xb, int64_t xe, int64_t n, int d,
+    const float* __restrict__ qb32, const float* __restrict__ db32, const float* __restrict__ p32,
+    const float* __restrict__ ge32, float scale, int64_t seg_len, int P, int S, Entry* __restrict__ part,
+    double* __restrict__ blockstats, int VEC4, int STATS, CertArgs cert, unsigned int* __restrict__ rowthr) {
+    int64_t panel, seg;
+    sweep_block(blockIdx.x, P, S, panel, seg);
+    if (panel >= P || seg >= S) return;  // grid padding (uniform per workgroup, before any barrier)
+    __shared__ float sY[2][BY * STR];    // two chunks of Y tiles, 32 features each
+    __shared__ double sQB64[ST ? BX : 1], sDB64[2][ST ? BY : 1];
+    __shared__ float sDB[2][BY];
+    __shared__ float sGE[2][BY];
+    __shared__ Entry sQ[256 * (QN + 1)];
+    __shared__ double sRed[4][5];
+
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = tid >> 6;
+    const int h = lane >> 5;
+    const int r = lane & 31;
+    const int64_t rows = xe - xb;
+    const int64_t x0 = xb + panel * BX;
+    const int64_t y_begin = seg * seg_len;
+    const int64_t y_end = (y_begin + seg_len < n) ? (y_begin + seg_len) : n;
+    SweepRow<K1> s;
+    sweep_row_init<K1, false>(s, x0 + wave * 32 + r, xe, STATS, qb32, p32, nullptr);
+    const float slack = row_cert_slack(STATS, cert, s.row, s.ok, scale);
+    if (ST && tid < BX) sQB64[tid] = (STATS && x0 + tid < xe) ? cert.qb[x0 + tid] : 0.0;
+
+    // four features of a row from feature k on (zeros beyond the row's d features, or for a row that is not there)
+    auto quad = [&](const float* base, bool ok, int k) {
+        float4 v = make_float4(0, 0, 0, 0);
+        if (VEC4) {
+            if (ok && k < d) v = *reinterpret_cast<const float4*>(base + k);
+        } else if (ok) {
+            if (k < d) v.x = base[k];
+            if (k + 1 < d) v.y = base[k + 1];
+            if (k + 2 < d) v.z = base[k + 2];
+            if (k + 3 < d) v.w = base[k + 3];
+        }
+        return v;
+    };
+    // B operand: this lane's X row, features h*16 .. h*16+15 of each chunk
+    float4 bx[NC][4];
+#pragma unroll
+    for (int c = 0; c < NC; ++c)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) bx[c][g] = quad(X + s.row * d, s.ok, c * KC + h * 16 + 4 * g);
+
+    float4 gy[4];       // the next chunk of Y, and at a tile's first chunk its biases
+    float gdb = 0.0f, gge = 0.0f;
+    double gdb64 = 0.0;
+    auto load = [&](int64_t ytile, int c) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int lin = tid + 256 * i;
+            const int64_t yr = ytile + (lin >> 3);
+            gy[i] = quad(Y + yr * d, yr < y_end, c * KC + 4 * (lin & 7));
+        }
+        if (c == 0 && tid < BY) {
+            const int64_t j = ytile + tid;
+            gdb = j < y_end ? db32[j] : 0.0f;
+            if (ST) {
+                gge = (STATS && j < y_end) ? ge32[j] : 0.0f;
+                gdb64 = (STATS && j < y_end) ? cert.db[j] : 0.0;
+            }
+        }
+    };
+    // into stage `at`; the biases into set `set`
+    auto store = [&](int at, int set, int c) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int lin = tid + 256 * i;
+            *reinterpret_cast<float4*>(&sY[at][(lin >> 3) * STR + 4 * (lin & 7)]) = gy[i];
+        }
+        if (c == 0 && tid < BY) {
+            sDB[set][tid] = gdb;
+            if (ST) {
+                sGE[set][tid] = gge;
+                sDB64[set][tid] = gdb64;
+            }
+        }
+    };
+    v16f acc[NB];
+    auto compute = [&](int at, int c, const float4 (&b4)[4]) {
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            if (c * KC + 4 * g >= d) break;  // (lane halves hold features 4 g and 16 + 4 g on: zeros both)
+            const float4 bv = b4[g];
+            float4 av[NB];
+#pragma unroll
+            for (int b = 0; b < NB; ++b)
+                av[b] = *reinterpret_cast<const float4*>(&sY[at][(b * 32 + r) * STR + h * 16 + 4 * g]);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+#pragma unroll
+                for (int b = 0; b < NB; ++b) {
+                    const float ae = e == 0 ? av[b].x : e == 1 ? av[b].y : e == 2 ? av[b].z : av[b].w;
+                    const float be = e == 0 ? bv.x : e == 1 ? bv.y : e == 2 ? bv.z : bv.w;
+                    acc[b] = __builtin_amdgcn_mfma_f32_32x32x2f32(ae, be, acc[b], 0, 0, 0);
+                }
+            }
+        }
+    };
+
+    load(y_begin, 0);
+    store(0, 0, 0);
+    __syncthreads();
+    int at = 0, set = 0;
+    for (int64_t ytile = y_begin; ytile < y_end; ytile += BY) {
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
+#pragma unroll
+            for (int q = 0; q < 16; ++q) acc[b][q] = 0.0f;
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+            const bool last = c + 1 == NC;
+            load(last ? ytile + BY : ytile, last ? 0 : c + 1);  // (past the segment: zeros)
+            compute(at, c, bx[c]);
+            if (last) {
+                // the epilogue keeps its own barrier out (its biases have two sets, its queue is per lane)
+#define HM_EPILOGUE(FULL_TILE)                                                                                         \
+    sweep_epilogue<K1, false, false, BY, FULL_TILE, ST, false, false>(                                                 \
+        acc, s, tid, wave, h, r, ytile, y_end, x0, panel, n, scale, STATS, slack, sQB64, sDB64[set], sDB[set], sGE[set], \
+        nullptr, nullptr, nullptr, nullptr, nullptr, 0, rowthr, xb, sQ)
+                if (y_end - ytile >= (int64_t)(NB * 32) && x0 + BX <= xe) HM_EPILOGUE(true);
+                else HM_EPILOGUE(false);
+#undef HM_EPILOGUE
+            }
+            store(at ^ 1, set ^ 1, last ? 0 : c + 1);
+            __syncthreads();  // publishes the next chunk and retires all reads of this one
+            at ^= 1;
+        }
+        set ^= 1;
+    }
+    sweep_finish<K1, false>(s, tid, lane, wave, h, seg, rows, xb, P, panel, STATS, part, blockstats, sRed);
 }
 
 // -------------------------------------------------------------------------------------------------
@@ -2874,7 +3020,8 @@ inline int64_t chunk_rows(int64_t m, int64_t n, int kl, bool fused, int bx, int6
 
 // Y segments per sweep launch: enough workgroups to fill the chip (SWEEP_WGS), and for k > 2 at least 8 so each
 // row has 16 partial lists; at most `cap`, and segments of at least `min_tiles` tiles (4 amortise a workgroup's
-// start; the wide pass, whose few gathered rows make it latency-bound, takes 1). Among up to twice that many
+// start; the wide pass, whose few gathered rows make it latency-bound, takes 1), shorter ones where those would leave
+// CUs without a workgroup (2048 x 2048: 16 panels of 4 segments kept 64 of the 256 CUs busy). Among up to twice that many
 // segments the first whose workgroups fill whole rounds of the CUs (within 3%) is taken: a partial last round
 // idles CUs.
 inline int choose_segments(int64_t m, int64_t n, int k, int cap, int bx, int min_tiles = 4) {
@@ -2883,6 +3030,8 @@ inline int choose_segments(int64_t m, int64_t n, int k, int cap, int bx, int min
     int64_t s = (SWEEP_WGS + panels - 1) / panels;
     if (k > 2 && s < 8) s = 8;
     int64_t max_s = tiles / min_tiles > 0 ? tiles / min_tiles : 1;
+    const int64_t fill = (SWEEP_CUS + panels - 1) / panels;
+    if (max_s < fill) max_s = fill < tiles ? fill : tiles;
     if (max_s > cap) max_s = cap;
     if (s > max_s) s = max_s;
     if (s < 1) s = 1;
@@ -3224,6 +3373,12 @@ int run_bidir(hipStream_t st, const float* X, const float* Y, int64_t m, int64_t
                            st, rowthr, rows, neg_inf_key);
         HM_LAUNCH_CHECK("fill_u32");
 #define NOWIDE (const float*)nullptr, (int*)nullptr, (int*)nullptr, 0
+// up to 64 features: two workgroups on a CU (60001 x 60001 points, d = 4, with the certificate 12.5 -> 9.4 ms, without
+// 5.5 -> 4.1)
+#define HM_SHORT(NC, ST)                                                                                             \
+    hipLaunchKernelGGL((l2sq_sweep_short<K1, NC, ST>), grid, dim3(256), 0, st, X, Y, xb, xe, n, d, qb32, db32, p32,  \
+                       ge32, (float)scale, plan.seg_len, (int)panels, plan.S, part, blockstats, (int)vec4,           \
+                       (int)want_stats, cert, rowthr)
 #define HM_SWEEP(TL, CL, ST)                                                                                         \
     do {                                                                                                             \
         if (i8)                                                                                                      \
@@ -3240,6 +3395,10 @@ int run_bidir(hipStream_t st, const float* X, const float* Y, int64_t m, int64_t
                                sd, ld,                                                                               \
                                qb32, db32, p32, ge32, (float)scale, plan.seg_len, (int)panels, plan.S, part,         \
                                colpart, colthr, blockstats, (int)want_stats, cert, NOWIDE, rowthr);                 \
+        else if (!CL && d <= KC)                                                                                     \
+            HM_SHORT(1, ST);                                                                                         \
+        else if (!CL && d <= 2 * KC)                                                                                 \
+            HM_SHORT(2, ST);                                                                                         \
         else                                                                                                         \
             hipLaunchKernelGGL((l2sq_sweep<K1, TL, CL, false, ST>), grid, dim3(256), 0, st, X, Y, xb, xe, n, d, d,   \
                                qb32,                                                                                 \
@@ -3267,6 +3426,7 @@ int run_bidir(hipStream_t st, const float* X, const float* Y, int64_t m, int64_t
         }
         prof_end(st);
 #undef HM_SWEEP
+#undef HM_SHORT
         HM_LAUNCH_CHECK("l2sq_sweep");
         if (want_stats) {
             hipLaunchKernelGGL(l2sq_reduce_stats, dim3(1), dim3(256), 0, st, blockstats, (int64_t)panels * plan.S,
@@ -3346,6 +3506,10 @@ int run_bidir(hipStream_t st, const float* X, const float* Y, int64_t m, int64_t
                 hipLaunchKernelGGL(fill_u32, tgrid, dim3(256), 0, st, rowthr, rows,
                                    0x007fffffu /* float_key(-INFINITY) */);
             HM_LAUNCH_CHECK("row thresholds");
+#define HM_SHORT2(NC)                                                                                                \
+    hipLaunchKernelGGL((l2sq_sweep_short<K1, NC, false>), grid, dim3(256), 0, st, Y, X, yb, ye, m, d, db32, qb32,    \
+                       ge32, p32, (float)scale, plan2.seg_len, (int)panels2, plan2.S, part, blockstats, (int)vec4,   \
+                       0, CertArgs{}, rowthr)
 #define HM_SWEEP2(TL)                                                                                                \
     do {                                                                                                             \
         if (i8)                                                                                                      \
@@ -3360,6 +3524,10 @@ int run_bidir(hipStream_t st, const float* X, const float* Y, int64_t m, int64_t
             hipLaunchKernelGGL((l2sq_sweep_split<K1, false>), grid, dim3(256), 0, st, SYc, SX, yb, ye, m, sd, \
                                ld, db32, qb32, ge32, p32, (float)scale, plan2.seg_len, (int)panels2, plan2.S, part,  \
                                colpart, colthr, blockstats, 0, CertArgs{}, NOWIDE, rowthr);                         \
+        else if (d <= KC)                                                                                            \
+            HM_SHORT2(1);                                                                                            \
+        else if (d <= 2 * KC)                                                                                        \
+            HM_SHORT2(2);                                                                                            \
         else                                                                                                         \
             hipLaunchKernelGGL((l2sq_sweep<K1, TL, false>), grid, dim3(256), 0, st, Y, X, yb, ye, m, d, d, db32,     \
                                qb32, ge32, p32, (float)scale, plan2.seg_len, (int)panels2, plan2.S, part, colpart,   \
@@ -3370,6 +3538,7 @@ int run_bidir(hipStream_t st, const float* X, const float* Y, int64_t m, int64_t
             else HM_SWEEP2(false);
             prof_end(st);
 #undef HM_SWEEP2
+#undef HM_SHORT2
 #undef NOWIDE
             HM_LAUNCH_CHECK("l2sq_sweep");
             hipLaunchKernelGGL(zero_words, dim3(1), dim3(64), 0, st, reinterpret_cast<unsigned long long*>(redo_count), 1);

@@ -151,6 +151,23 @@ def test_l2sq_chunked_sides_and_ties(cuda, m, n, d, k, integer, precision):
     assert_l2sq_certificate(st, l2sq_certificate_bounds(X, Y, p, q, qb, db))
 
 
+@pytest.mark.parametrize("d", [1, 4, 15, 16, 17, 32, 33, 36, 63, 64, 65])
+@pytest.mark.parametrize("m,n,k", [(129, 257, 1), (700, 3, 2), (385, 1100, 8), (130, 2049, 16)])
+def test_l2sq_few_features_match_oracle(cuda, d, m, n, k):
+    """The fp32 sweep of up to 64 features at the edges of its chunks, operand halves and tiles (65: the general
+    sweep), rows, columns and certificate, and rows alone (the sweep without the certificate)."""
+    X, Y, p, q, qb, db = _l2sq_case(m, n, d, 31 * d + k, dup=True)
+    orv, ori, ocv, oci, _ = oracle.l2sq_scan(X, Y, p, q, qb, db, k, 2.0)
+    t = _to(cuda, X, Y, p, q, qb, db)
+    rv, ri, cv, ci, st = pricing_l2sq(*t, k, linf=True, precision="fp32")
+    for got, want in ((rv, orv), (ri, ori), (cv, ocv), (ci, oci)):
+        np.testing.assert_array_equal(got.cpu().numpy(), want)
+    assert_l2sq_certificate(st, l2sq_certificate_bounds(X, Y, p, q, qb, db))
+    rv, ri, _, _, _ = pricing_l2sq(*t, k, cols=False, stats=False, precision="fp32")
+    np.testing.assert_array_equal(rv.cpu().numpy(), orv)
+    np.testing.assert_array_equal(ri.cpu().numpy(), ori)
+
+
 @pytest.mark.parametrize("side", ["x", "y"])
 @pytest.mark.parametrize("d", [5, 256])
 @pytest.mark.parametrize("precision", ["fp32", "bf16x3", "int8x3"])
