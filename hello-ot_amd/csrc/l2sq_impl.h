@@ -126,21 +126,30 @@ constexpr float CERT_REL = 1.4901161e-07f;
 // slack are decided in fp32 (a positive one adds sg^2 to the tile's fp32 sum); pairs within it get sigma' in fp64,
 // which decides the count and adds sigma'^2 to the lane's fp64 sum.
 //
-// cert_fast is the per-pair part, without branches: the cost terms, the fp32 decision, and `near` set for a pair
-// within the slack. A tile with a near pair on some lane runs cert_near over its pairs afterwards (rare: the slack is
-// a few fp32 units of the row's largest score).
-__device__ __forceinline__ void cert_fast(bool ok, float w, float ge, float pi, float qbi, float slack, float& tden,
-                                          float& cmax, float& tnum, unsigned int& tcnt, bool& near) {
+// cert_cost and cert_score (cert_fast: both) are the per-pair part, without branches: the cost terms; the fp32 decision
+// and `near`, set for a pair within the slack. A tile with a near pair on some lane runs cert_near over its pairs
+// afterwards (rare: the slack is a few fp32 units of the row's largest score). The 128-row sweeps vote per group of four
+// pairs a lane and skip cert_score, half of the part's instructions, where the wave holds neither kind of pair (near the
+// optimum one pair in ten thousand is violated, one group in thirty).
+__device__ __forceinline__ void cert_cost(bool ok, float w, float ge, float pi, float& tden, float& cmax) {
     const float cost = (pi + ge) - w;
     const float cm = ok ? cost : 0.0f;
     tden = fmaf(cm, cm, tden);
     cmax = fmaxf(cmax, fabsf(cm));
+}
+__device__ __forceinline__ void cert_score(bool ok, float w, float qbi, float slack, float& tnum, unsigned int& tcnt,
+                                           bool& near) {
     const float sg = w + qbi;
     const bool pos = ok && sg > slack;
     const float sp = pos ? sg : 0.0f;
     tnum = fmaf(sp, sp, tnum);
     tcnt += pos ? 1u : 0u;
     near = near || (ok && fabsf(sg) <= slack);
+}
+__device__ __forceinline__ void cert_fast(bool ok, float w, float ge, float pi, float qbi, float slack, float& tden,
+                                          float& cmax, float& tnum, unsigned int& tcnt, bool& near) {
+    cert_cost(ok, w, ge, pi, tden, cmax);
+    cert_score(ok, w, qbi, slack, tnum, tcnt, near);
 }
 
 __device__ __forceinline__ void cert_near(bool ok, float t, float w, float qbi, float slack, float scale, double qb64,
@@ -534,9 +543,13 @@ __device__ __forceinline__ void sweep_row_init(SweepRow<K1>& s, int64_t row, int
 // w = scale*dot + db into the row list (or appends for the wide pass), adds the certificate terms and, with COLS,
 // passes the tile's scores scale*dot + qb through LDS so that each Y row keeps its best K1 over the workgroup's
 // 128 X rows, CPASS Y rows at a time (sC holds CPASS * CST floats; 256 / CPASS threads scan each row and merge
-// their lists). Ends with a barrier, so that the next tile may rewrite sDB / sGE / sC (SYNC; a sweep that keeps two
-// sets of them and no columns has its own barrier per tile).
-template <int K1, bool COLS, bool APPEND, int CPASS, bool FULL, bool ST, bool SRT = false, bool SYNC = true>
+// their lists). Ends with a barrier, so that the next tile may rewrite sDB / sGE / sC.
+// LANES (with FULL, without columns; l2sq_sweep_short, l2sq_sweep_split) takes ragged tiles and panels without a per-pair test: Y rows
+// beyond the segment have the bias -inf, which no list, vote or decision lets through (only the cost sums test the
+// limit, in ragged tiles), the caller drops the sums of lanes beyond the panel, and has its own barrier per tile. A second
+// copy for ragged tiles made the compiler keep its 64 limit tests and spill 150 to 400 vectors a lane: 60001 x 60001, d = 4,
+// with the certificate 9.4 ms with it, 4.3 without; 65536 x 131072, d = 64 (split copies) 8.3 and 7.1.
+template <int K1, bool COLS, bool APPEND, int CPASS, bool FULL, bool ST, bool SRT = false, bool LANES = false>
 __device__ __forceinline__ void sweep_epilogue(const v16f (&tot)[NB], SweepRow<K1>& s, int tid, int wave, int h,
                                                int r, int64_t ytile, int64_t y_end, int64_t x0, int64_t panel,
                                                int64_t n, float scale, int STATS_, float slack, const double* sQB64,
@@ -559,8 +572,8 @@ __device__ __forceinline__ void sweep_epilogue(const v16f (&tot)[NB], SweepRow<K
     const bool rok = FULL || s.ok;
     // the row's shared threshold: scores at or below it cannot enter the row's merged lists (row_threshold_*);
     // with SRT, sRT holds the panel's thresholds as read at the start of the tile
-    float rthr = -INFINITY;
-    if (!APPEND && rok && rowthr) {
+    float rthr = LANES && !s.ok ? INFINITY : -INFINITY;
+    if (!APPEND && (LANES ? s.ok : rok) && rowthr) {
         if constexpr (SRT) rthr = key_float(sRT[wave * 32 + r]);
         else rthr = row_threshold_get(rowthr, s.row - xb);
     }
@@ -599,7 +612,29 @@ __device__ __forceinline__ void sweep_epilogue(const v16f (&tot)[NB], SweepRow<K
                 } else {
                     amax = fmaxf(amax, ok ? w : -INFINITY);
                 }
-                if (STATS) cert_fast(ok, w, ges[cc], s.pi, s.qbi, slack, tden, s.cmax, tnum, tcnt, near);
+                if (STATS && !LANES) cert_cost(ok, w, ges[cc], s.pi, tden, s.cmax);
+            }
+            if (STATS && LANES) {
+                if (y_end - ytile >= (int64_t)(NB * 32)) {
+#pragma unroll
+                    for (int cc = 0; cc < 4; ++cc)
+                        cert_cost(true, fmaf(scale, tot[b][4 * a + cc], dbs[cc]), ges[cc], s.pi, tden, s.cmax);
+                } else {
+#pragma unroll
+                    for (int cc = 0; cc < 4; ++cc)
+                        cert_cost(ytile + jl0 + cc < y_end, fmaf(scale, tot[b][4 * a + cc], dbs[cc]), ges[cc], s.pi, tden,
+                                  s.cmax);
+                }
+            }
+            // rounding is monotone, so amax + qb is the group's largest score: unless some lane's reaches -slack the
+            // group has neither a violated nor a near pair
+            if (STATS && __any(amax + s.qbi >= -slack)) {
+#pragma unroll
+                for (int cc = 0; cc < 4; ++cc) {
+                    const float w = fmaf(scale, tot[b][4 * a + cc], dbs[cc]);
+                    const bool ok = rok && (FULL || 4 * h < ylim - (b * 32 + 8 * a + cc));
+                    cert_score(ok, w, s.qbi, slack, tnum, tcnt, near);
+                }
             }
             if (!APPEND && __any(amax > qthr)) {
                 // every score above the threshold, in pair order, as if each had been tested
@@ -716,7 +751,7 @@ __device__ __forceinline__ void sweep_epilogue(const v16f (&tot)[NB], SweepRow<K
             }
         }
     }
-    if (SYNC) __syncthreads();  // all epilogue reads of sDB/sGE/sC finish before the next tile rewrites them
+    if (!LANES) __syncthreads();  // all epilogue reads of sDB/sGE/sC finish before the next tile rewrites them
 }
 
 // End of a sweep workgroup: lane lists -> part[(seg*rows + local row)*2 + h][K1], certificate partials reduced
@@ -1035,7 +1070,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void l
         }
         if (c == 0 && tid < BY) {
             const int64_t j = ytile + tid;
-            gdb = j < y_end ? db32[j] : 0.0f;
+            gdb = j < y_end ? db32[j] : -INFINITY;
             if (ST) {
                 gge = (STATS && j < y_end) ? ge32[j] : 0.0f;
                 gdb64 = (STATS && j < y_end) ? cert.db[j] : 0.0;
@@ -1061,19 +1096,20 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void l
     auto compute = [&](int at, int c, const float4 (&b4)[4]) {
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
-            if (c * KC + 4 * g >= d) break;  // (lane halves hold features 4 g and 16 + 4 g on: zeros both)
-            const float4 bv = b4[g];
-            float4 av[NB];
+            if (c * KC + 4 * g < d) {  // (else both lane halves' features, 4 g and 16 + 4 g on, are zeros)
+                const float4 bv = b4[g];
+                float4 av[NB];
 #pragma unroll
-            for (int b = 0; b < NB; ++b)
-                av[b] = *reinterpret_cast<const float4*>(&sY[at][(b * 32 + r) * STR + h * 16 + 4 * g]);
+                for (int b = 0; b < NB; ++b)
+                    av[b] = *reinterpret_cast<const float4*>(&sY[at][(b * 32 + r) * STR + h * 16 + 4 * g]);
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
+                for (int e = 0; e < 4; ++e) {
 #pragma unroll
-                for (int b = 0; b < NB; ++b) {
-                    const float ae = e == 0 ? av[b].x : e == 1 ? av[b].y : e == 2 ? av[b].z : av[b].w;
-                    const float be = e == 0 ? bv.x : e == 1 ? bv.y : e == 2 ? bv.z : bv.w;
-                    acc[b] = __builtin_amdgcn_mfma_f32_32x32x2f32(ae, be, acc[b], 0, 0, 0);
+                    for (int b = 0; b < NB; ++b) {
+                        const float ae = e == 0 ? av[b].x : e == 1 ? av[b].y : e == 2 ? av[b].z : av[b].w;
+                        const float be = e == 0 ? bv.x : e == 1 ? bv.y : e == 2 ? bv.z : bv.w;
+                        acc[b] = __builtin_amdgcn_mfma_f32_32x32x2f32(ae, be, acc[b], 0, 0, 0);
+                    }
                 }
             }
         }
@@ -1093,21 +1129,21 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void l
             const bool last = c + 1 == NC;
             load(last ? ytile + BY : ytile, last ? 0 : c + 1);  // (past the segment: zeros)
             compute(at, c, bx[c]);
-            if (last) {
-                // the epilogue keeps its own barrier out (its biases have two sets, its queue is per lane)
-#define HM_EPILOGUE(FULL_TILE)                                                                                         \
-    sweep_epilogue<K1, false, false, BY, FULL_TILE, ST, false, false>(                                                 \
-        acc, s, tid, wave, h, r, ytile, y_end, x0, panel, n, scale, STATS, slack, sQB64, sDB64[set], sDB[set], sGE[set], \
-        nullptr, nullptr, nullptr, nullptr, nullptr, 0, rowthr, xb, sQ)
-                if (y_end - ytile >= (int64_t)(NB * 32) && x0 + BX <= xe) HM_EPILOGUE(true);
-                else HM_EPILOGUE(false);
-#undef HM_EPILOGUE
-            }
             store(at ^ 1, set ^ 1, last ? 0 : c + 1);
+            if (last) {
+                sweep_epilogue<K1, false, false, BY, true, ST, false, true>(
+                    acc, s, tid, wave, h, r, ytile, y_end, x0, panel, n, scale, STATS, slack, sQB64, sDB64[set], sDB[set],
+                    sGE[set], nullptr, nullptr, nullptr, nullptr, nullptr, 0, rowthr, xb, sQ);
+            }
             __syncthreads();  // publishes the next chunk and retires all reads of this one
             at ^= 1;
         }
         set ^= 1;
+    }
+    if (!s.ok) {  // lanes beyond the panel
+        s.num64 = s.den64 = 0.0;
+        s.cnt = 0u;
+        s.cmax = 0.0f;
     }
     sweep_finish<K1, false>(s, tid, lane, wave, h, seg, rows, xb, P, panel, STATS, part, blockstats, sRed);
 }
@@ -1419,6 +1455,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(COLS ? 1 : 
             step(I2{});
             step(I3{});
         }
+        if constexpr (!COLS && !APPEND) {
+            if (y_end - ytile < (int64_t)BY) {  // (LANES: the bias of the columns past the segment)
+                if (tid < BY && ytile + tid >= y_end) sDB[tid] = -INFINITY;
+                __syncthreads();
+            }
+            sweep_epilogue<K1, false, false, BY, true, ST, true, true>(
+                acc, s, tid, wave, h, r, ytile, y_end, x0, panel, n, scale, STATS, slack, sQB64, sDB64, sDB, sGE, nullptr,
+                nullptr, nullptr, nullptr, nullptr, 0, rowthr, xb, sQ, sRT);
+            __syncthreads();  // its reads of sDB and sGE finish before the next tile's loads rewrite them
+        } else {
 #define HM_EPILOGUE(FULL_TILE)                                                                                  \
     sweep_epilogue<K1, COLS, APPEND, BY, FULL_TILE, ST, true>(acc, s, tid, wave, h, r, ytile, y_end, x0, panel, n,   \
                                                    scale, STATS, slack, sQB64, sDB64, sDB, sGE, sC, colpart,     \
@@ -1427,8 +1473,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(COLS ? 1 : 
         if (y_end - ytile >= (int64_t)(NB * 32) && x0 + BX <= xe) HM_EPILOGUE(true);
         else HM_EPILOGUE(false);
 #undef HM_EPILOGUE
+        }
     }
     wait_vmcnt<0>();  // the loads ahead into LDS land before the workgroup can end
+    if (!COLS && !APPEND && !s.ok) {  // lanes beyond the panel
+        s.num64 = s.den64 = 0.0;
+        s.cnt = 0u;
+        s.cmax = 0.0f;
+    }
     sweep_finish<K1, APPEND>(s, tid, lane, wave, h, seg, rows, xb, P, panel, STATS, part, blockstats, sRed);
 }
 
@@ -2942,19 +2994,16 @@ __global__ void running_floor(double* __restrict__ out, int64_t n, const double*
     }
 }
 
-__global__ void exact_row_max(const double* __restrict__ row_val, int64_t m, int k, double* __restrict__ stats) {
-    __shared__ double s[256];
+__global__ __launch_bounds__(256) void exact_row_max(const double* __restrict__ row_val, int64_t m, int k,
+                                                     double* __restrict__ stats) {
     double v = 0.0;
-    for (int64_t i = threadIdx.x; i < m; i += 256) v = fmax(v, row_val[i * k]);
-    s[threadIdx.x] = v;
-    __syncthreads();
-    for (int w = 128; w >= 1; w >>= 1) {
-        if ((int)threadIdx.x < w) s[threadIdx.x] = fmax(s[threadIdx.x], s[threadIdx.x + w]);
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) stats[3] = s[0];
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < m; i += (int64_t)gridDim.x * 256)
+        v = fmax(v, row_val[i * k]);
+    for (int o = 32; o >= 1; o >>= 1) v = fmax(v, __shfl_xor(v, o, 64));
+    // (stats[3] is 0 before this launch, and positive doubles order like their bits)
+    if ((threadIdx.x & 63) == 0 && v > 0.0)
+        atomicMax(reinterpret_cast<unsigned long long*>(stats + 3), (unsigned long long)__double_as_longlong(v));
 }
-
 __global__ void zero_words(unsigned long long* p, int count) {
     if ((int)threadIdx.x < count) p[threadIdx.x] = 0ull;
 }
@@ -3373,8 +3422,8 @@ int run_bidir(hipStream_t st, const float* X, const float* Y, int64_t m, int64_t
                            st, rowthr, rows, neg_inf_key);
         HM_LAUNCH_CHECK("fill_u32");
 #define NOWIDE (const float*)nullptr, (int*)nullptr, (int*)nullptr, 0
-// up to 64 features: two workgroups on a CU (60001 x 60001 points, d = 4, with the certificate 12.5 -> 9.4 ms, without
-// 5.5 -> 4.1)
+// up to 64 features: two workgroups on a CU and one copy of the epilogue (60001 x 60001 points, d = 4, with the
+// certificate 12.5 -> 4.3 ms, without 5.5 -> 1.9)
 #define HM_SHORT(NC, ST)                                                                                             \
     hipLaunchKernelGGL((l2sq_sweep_short<K1, NC, ST>), grid, dim3(256), 0, st, X, Y, xb, xe, n, d, qb32, db32, p32,  \
                        ge32, (float)scale, plan.seg_len, (int)panels, plan.S, part, blockstats, (int)vec4,           \
@@ -3559,7 +3608,9 @@ int run_bidir(hipStream_t st, const float* X, const float* Y, int64_t m, int64_t
     }
     if (want_stats) {
         if (!want_rows) return fail(HM_EINVAL, "l2sq pricing: the certificate needs the row lists");
-        hipLaunchKernelGGL(exact_row_max, dim3(1), dim3(256), 0, st, row_val, m, k, stats);
+        // (one workgroup took 160 us at 131072 rows)
+        hipLaunchKernelGGL(exact_row_max, dim3((unsigned)((m + 1023) / 1024 < 256 ? (m + 1023) / 1024 : 256)), dim3(256),
+                           0, st, row_val, m, k, stats);
         HM_LAUNCH_CHECK("exact_row_max");
     }
     return HM_OK;
