@@ -684,8 +684,9 @@ __device__ __forceinline__ void sweep_epilogue(const v16f (&tot)[NB], SweepRow<K
             for (int q = 0; q < 16; ++q) {
                 const int jl = b * 32 + 8 * (q / 4) + 4 * h + (q % 4);
                 const float t = tot[b][q];
-                cert_near(rok && (FULL || 4 * h < ylim - (jl - 4 * h)), t, fmaf(scale, t, sDB[jl]), s.qbi, slack, scale, qb64,
-                          sDB64[jl], tcnt, s.num64);
+                // (LANES: an infinite slack, from a dual beyond fp32, would let the columns past the segment through)
+                const bool in = LANES ? sDB[jl] > -INFINITY : FULL || 4 * h < ylim - (jl - 4 * h);
+                cert_near(rok && in, t, fmaf(scale, t, sDB[jl]), s.qbi, slack, scale, qb64, sDB64[jl], tcnt, s.num64);
             }
         }
     }

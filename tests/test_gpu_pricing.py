@@ -168,6 +168,20 @@ def test_l2sq_few_features_match_oracle(cuda, d, m, n, k):
     np.testing.assert_array_equal(ri.cpu().numpy(), ori)
 
 
+@pytest.mark.parametrize("d,precision", [(5, "fp32"), (40, "fp32"), (5, "bf16x3"), (100, "bf16x3")])
+def test_l2sq_count_with_a_dual_beyond_fp32(cuda, d, precision):
+    """One column bias that fp32 holds as -inf makes every row's certificate slack infinite, so every pair's sign is
+    taken in fp64: the columns past the last tile's end are still not counted."""
+    X, Y, p, q, qb, db = _l2sq_case(130, 300, d, 7 * d)
+    db[7] = -1e50
+    sigma = 2.0 * X.astype(np.float64) @ Y.astype(np.float64).T + qb[:, None] + db
+    # the scores are 2 dots: fp32 sums of d products, or split products without lo * lo (2^-18) and the two lows' rounding
+    rel = (d + 2) * 2.0 ** -24 + (0 if precision == "fp32" else 3 * 2.0 ** -18)
+    near = 2.02 * rel * np.sqrt(p.max() * q.max())
+    st = pricing_l2sq(*_to(cuda, X, Y, p, q, qb, db), 1, rows=False, cols=False, stats=True, precision=precision)[4]
+    assert (sigma > near).sum() <= int(st[2]) <= (sigma > -near).sum()
+
+
 @pytest.mark.parametrize("side", ["x", "y"])
 @pytest.mark.parametrize("d", [5, 256])
 @pytest.mark.parametrize("precision", ["fp32", "bf16x3", "int8x3"])
