@@ -312,10 +312,10 @@ extern "C" int hm_sddmm_l2sq_csr(void* stream, const float* X, const float* Y, c
 #define HM_SDDMM(XR) \
     hipLaunchKernelGGL((sddmm_l2sq_csr_kernel<XR>), dim3(grid), dim3(256), 0, st, X, Y, p, q, rowptr, col, m, d, scale, out)
     prof_begin(st, "sddmm_l2sq_csr");
-    // level between 128 and 256 features (262144 rows of 16 entries, d = 256: 0.74 ms and 0.75 in fours, 5.7 TB/s of
-    // gathered rows); elsewhere the fours are ahead (30000 rows of 20, d = 1024: 0.69 -> 0.41 ms; 60000 rows of 20,
-    // d = 128: 0.19 -> 0.12)
-    if (quad_rows(X, Y, d) && (d <= 128 || d > 256))
+    // from 129 to 512 features a wave per entry with x in registers is level or ahead (262144 rows of 16 entries, d = 256:
+    // 0.74 ms and 0.75 in fours, 5.7 TB/s of gathered rows; 105 thousand rows of 20, d = 512: 0.72 and 0.81); elsewhere the
+    // fours are (89 thousand rows of 20, d = 600: 1.26 -> 0.84 ms; 120 thousand rows of 20, d = 128: 0.47 -> 0.33)
+    if (quad_rows(X, Y, d) && (d <= 128 || d > 512))
         hipLaunchKernelGGL(sddmm_quad_kernel, dim3(grid), dim3(256), 0, st, X, Y, p, q, rowptr, col, m, d, scale, out);
     else if (d <= 64) HM_SDDMM(1);
     else if (d <= 128) HM_SDDMM(2);
@@ -340,7 +340,7 @@ extern "C" int hm_pair_costs_l2sq(void* stream, const float* X, const float* Y, 
 #define HM_PAIRS(GG)                                                                                            \
     hipLaunchKernelGGL((pair_costs_l2sq_kernel<GG>), dim3(grid_for(count, 256 / GG)), dim3(256), 0, st, X, Y, p, q, \
                        rows, cols, count, d, scale, out)
-    // (up to 16 features the groups below use more of their lanes)
+    // (up to 16 features the groups below use more of their lanes: level; 2 million pairs, d = 24: 0.30 -> 0.27 ms)
     if (d > 16 && quad_rows(X, Y, d))
         hipLaunchKernelGGL(pair_costs_quad_kernel, dim3(grid_for(count, 16)), dim3(256), 0, st, X, Y, p, q, rows, cols,
                            count, d, scale, out);
@@ -370,7 +370,8 @@ extern "C" int hm_pair_costs_norm(void* stream, const float* X, const float* Y, 
         else if (kind == HM_COST_LINF) HM_NORM(GG, HM_COST_LINF); \
         else HM_NORM(GG, HM_COST_L2);                        \
     } while (0)
-    if (d > 16 && quad_rows(X, Y, d)) {
+    // (up to 32 features the groups below are ahead: 2 million pairs, l1, d = 24: 0.24 ms and 0.27 in fours; d = 40: 0.38 and 0.27)
+    if (d > 32 && quad_rows(X, Y, d)) {
 #define HM_NORM_QUAD(KK)                                                                                               \
     hipLaunchKernelGGL((pair_costs_norm_quad_kernel<KK>), dim3(grid_for(count, 16)), dim3(256), 0, st, X, Y, rows, cols, \
                        count, d, out)
