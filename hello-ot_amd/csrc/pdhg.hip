@@ -236,26 +236,55 @@ __global__ void k_fill_i32(int32_t* p, int64_t count, int32_t v) {
         p[i] = v;
 }
 
+// sums[key] += v over the wave's lanes with key >= 0, called by whole waves. Supports come with their edges in source order,
+// so neighbouring lanes often hold the same key, and their atomics to one word would queue: where the wave has few runs of
+// equal keys each run is summed by shuffles and added once (integers: the sums are the same). 12 million edges in source
+// order, 23 to a source: 685 us with an atomic per edge.
+template <typename T>
+__device__ __forceinline__ void add_runs(T* __restrict__ sums, int64_t key, T v) {
+    const int lane = threadIdx.x & 63;
+    const int64_t left = __shfl_up(key, 1, 64);
+    const unsigned long long heads = __ballot(lane == 0 || key != left);
+    if (__popcll(heads) > 24) {
+        if (key >= 0) atomicAdd(&sums[key], v);
+        return;
+    }
+    const int first = 63 - __clzll(heads & (~0ull >> (63 - lane)));  // the lane where this lane's run begins
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const T u = __shfl_up(v, o, 64);
+        if (lane - o >= first) v += u;
+    }
+    const bool last = lane == 63 || ((heads >> (lane + 1)) & 1ull);
+    if (last && key >= 0) atomicAdd(&sums[key], v);
+}
+
 // validation, degrees and the (node key, caller edge id) pairs of the incidence sort
 __global__ void k_edges(const int64_t* __restrict__ rows, const int64_t* __restrict__ cols, int64_t e, int64_t n,
                         int64_t nt, const int32_t* __restrict__ map_s, const int32_t* __restrict__ map_t,
                         int32_t* __restrict__ deg, uint32_t* __restrict__ keys, int32_t* __restrict__ vals,
                         int* __restrict__ flag) {
-    for (int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; j < e; j += (int64_t)gridDim.x * blockDim.x) {
-        const int64_t r = rows[j], c = cols[j];
-        if (r < 0 || r >= n || c < 0 || c >= nt) {
-            atomicOr(flag, 1);
-            keys[j] = 0;
-            keys[e + j] = (uint32_t)n;
-        } else {
-            const int64_t ri = map_s ? map_s[r] : r, ci = map_t ? map_t[c] : c;
-            atomicAdd(&deg[ri], 1);
-            atomicAdd(&deg[n + ci], 1);
-            keys[j] = (uint32_t)ri;
-            keys[e + j] = (uint32_t)(n + ci);
+    const int lane = threadIdx.x & 63;
+    for (int64_t j0 = (int64_t)blockIdx.x * blockDim.x + threadIdx.x - lane; j0 < e; j0 += (int64_t)gridDim.x * blockDim.x) {
+        const int64_t j = j0 + lane;
+        int64_t ri = -1, ci = -1;
+        if (j < e) {
+            const int64_t r = rows[j], c = cols[j];
+            if (r < 0 || r >= n || c < 0 || c >= nt) {
+                atomicOr(flag, 1);
+                keys[j] = 0;
+                keys[e + j] = (uint32_t)n;
+            } else {
+                ri = map_s ? map_s[r] : r;
+                ci = n + (map_t ? map_t[c] : c);
+                keys[j] = (uint32_t)ri;
+                keys[e + j] = (uint32_t)ci;
+            }
+            vals[j] = (int32_t)j;
+            vals[e + j] = (int32_t)j;
         }
-        vals[j] = (int32_t)j;
-        vals[e + j] = (int32_t)j;
+        add_runs(deg, ri, 1);
+        add_runs(deg, ci, 1);
     }
 }
 
@@ -311,31 +340,60 @@ __global__ void k_target_setup(const int32_t* __restrict__ eid, int64_t e, const
     }
 }
 
-// exclusive scan of deg[0..nodes) into off[0..nodes] with a single workgroup (setup only)
-__global__ void k_scan(const int32_t* __restrict__ deg, int64_t nodes, int32_t* __restrict__ off) {
-    __shared__ int64_t sums[1024];
-    const int t = threadIdx.x;
-    const int64_t per = (nodes + 1023) / 1024;
-    const int64_t b0 = t * per, b1 = (b0 + per < nodes) ? b0 + per : nodes;
+// Exclusive scan of deg[0..nodes) into off[0..nodes]: each workgroup scans `per` nodes, 1024 at a time, from the total of
+// the workgroups before it (part, of k_scan_sums; unused by a single workgroup). Latency bounds a scan by one workgroup
+// (1.8 ms at 2^20 nodes, each thread walking a run of its own), hence many above SCAN_ONE nodes.
+constexpr int SCAN_BLOCKS = 256;
+constexpr int64_t SCAN_ONE = 16384;  // up to here a second launch costs more than 16 rounds of one workgroup
+
+__global__ __launch_bounds__(1024) void k_scan_sums(const int32_t* __restrict__ deg, int64_t nodes, int64_t per,
+                                                    int64_t* __restrict__ part) {
+    __shared__ int64_t sums[16];
+    const int64_t b0 = blockIdx.x * per, b1 = (b0 + per < nodes) ? b0 + per : nodes;
     int64_t s = 0;
-    for (int64_t i = b0; i < b1; ++i) s += deg[i];
-    sums[t] = s;
+    for (int64_t i = b0 + threadIdx.x; i < b1; i += 1024) s += deg[i];
+    for (int o = 32; o >= 1; o >>= 1) s += __shfl_xor(s, o, 64);
+    if ((threadIdx.x & 63) == 0) sums[threadIdx.x >> 6] = s;
     __syncthreads();
-    if (t == 0) {
-        int64_t run = 0;
-        for (int i = 0; i < 1024; ++i) {
-            const int64_t v = sums[i];
-            sums[i] = run;
-            run += v;
+    if (threadIdx.x == 0) {
+        s = 0;
+        for (int w = 0; w < 16; ++w) s += sums[w];
+        part[blockIdx.x] = s;
+    }
+}
+
+__global__ __launch_bounds__(1024) void k_scan(const int32_t* __restrict__ deg, int64_t nodes, int64_t per,
+                                               const int64_t* __restrict__ part, int32_t* __restrict__ off) {
+    __shared__ int64_t sums[2][16];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int64_t b0 = blockIdx.x * per, b1 = (b0 + per < nodes) ? b0 + per : nodes;
+    if (b0 > 0 && b0 >= nodes) return;
+    int64_t run = threadIdx.x < blockIdx.x ? part[threadIdx.x] : 0;  // (SCAN_BLOCKS <= 1024)
+    for (int o = 32; o >= 1; o >>= 1) run += __shfl_xor(run, o, 64);
+    if (lane == 0) sums[1][wave] = run;
+    __syncthreads();
+    run = 0;
+    for (int w = 0; w < 16; ++w) run += sums[1][w];
+    int at = 0;
+    for (int64_t i0 = b0; i0 < b1; i0 += 1024, at ^= 1) {
+        const int64_t i = i0 + threadIdx.x;
+        const int64_t own = i < b1 ? deg[i] : 0;
+        int64_t v = own;
+        for (int o = 1; o < 64; o <<= 1) {
+            const int64_t u = __shfl_up(v, o, 64);
+            if (lane >= o) v += u;
         }
+        if (lane == 63) sums[at][wave] = v;
+        __syncthreads();  // (the other set is rewritten only after the next barrier)
+        int64_t before = run;
+        for (int w = 0; w < 16; ++w) {
+            const int64_t t = sums[at][w];
+            if (w < wave) before += t;
+            run += t;
+        }
+        if (i < b1) off[i] = (int32_t)(before + v - own);
     }
-    __syncthreads();
-    int64_t run = sums[t];
-    for (int64_t i = b0; i < b1; ++i) {
-        off[i] = (int32_t)run;
-        run += deg[i];
-    }
-    if (t == 1023) off[nodes] = (int32_t)run;  // the last range ends at `nodes`, so run is the total
+    if (b1 == nodes && threadIdx.x == 0) off[nodes] = (int32_t)run;
 }
 
 __global__ void k_node_setup(const int32_t* __restrict__ deg, const double* __restrict__ b,
@@ -366,14 +424,14 @@ __global__ void k_node_setup(const int32_t* __restrict__ deg, const double* __re
 // validation and the caller-numbered degrees
 __global__ void k_order_degrees(const int64_t* __restrict__ rows, const int64_t* __restrict__ cols, int64_t e,
                                 int64_t n, int64_t nt, int32_t* __restrict__ odeg, int* __restrict__ flag) {
-    for (int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; j < e; j += (int64_t)gridDim.x * blockDim.x) {
-        const int64_t r = rows[j], c = cols[j];
-        if (r < 0 || r >= n || c < 0 || c >= nt) {
-            atomicOr(flag, 1);
-        } else {
-            atomicAdd(&odeg[r], 1);
-            atomicAdd(&odeg[n + c], 1);
-        }
+    const int lane = threadIdx.x & 63;
+    for (int64_t j0 = (int64_t)blockIdx.x * blockDim.x + threadIdx.x - lane; j0 < e; j0 += (int64_t)gridDim.x * blockDim.x) {
+        const int64_t j = j0 + lane;
+        const int64_t r = j < e ? rows[j] : -1, c = j < e ? cols[j] : -1;
+        const bool ok = r >= 0 && r < n && c >= 0 && c < nt;
+        if (!ok && j < e) atomicOr(flag, 1);
+        add_runs(odeg, ok ? r : -1, 1);
+        add_runs(odeg, ok ? n + c : -1, 1);
     }
 }
 
@@ -397,10 +455,12 @@ __global__ void k_order_clear(unsigned long long* __restrict__ osum, int64_t cou
 __global__ void k_order_gather(const int64_t* __restrict__ rows, const int64_t* __restrict__ cols, int64_t e,
                                int64_t n, int to_sources, const uint32_t* __restrict__ ov,
                                unsigned long long* __restrict__ osum) {
-    for (int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; j < e; j += (int64_t)gridDim.x * blockDim.x) {
-        const int64_t r = rows[j], c = n + cols[j];
-        if (to_sources) atomicAdd(&osum[r], (unsigned long long)ov[c]);
-        else atomicAdd(&osum[c], (unsigned long long)ov[r]);
+    const int lane = threadIdx.x & 63;
+    for (int64_t j0 = (int64_t)blockIdx.x * blockDim.x + threadIdx.x - lane; j0 < e; j0 += (int64_t)gridDim.x * blockDim.x) {
+        const int64_t j = j0 + lane;
+        const int64_t r = j < e ? rows[j] : -1, c = j < e ? n + cols[j] : -1;
+        const int64_t from = to_sources ? c : r;
+        add_runs(osum, to_sources ? r : c, from >= 0 ? (unsigned long long)ov[from] : 0ull);
     }
 }
 
@@ -1120,7 +1180,12 @@ extern "C" int hm_pdhg_solve(void* stream, const int64_t* rows, const int64_t* c
     HM_HIP(hipMemcpyAsync(flag, P.flag, sizeof(flag), hipMemcpyDeviceToHost, st));
     HM_HIP(hipStreamSynchronize(st));
     if (flag[0]) return fail(HM_EINVAL, "active-support endpoint index is out of bounds");
-    hipLaunchKernelGGL(k_scan, dim3(1), dim3(1024), 0, st, P.deg, nodes, P.off);
+    const int scan_blocks = nodes > SCAN_ONE ? SCAN_BLOCKS : 1;
+    const int64_t scan_per = (nodes + scan_blocks - 1) / scan_blocks;
+    int64_t* const scan_part = reinterpret_cast<int64_t*>(P.partial);  // (RB * 4 words, free until the first norm)
+    if (scan_blocks > 1)
+        hipLaunchKernelGGL(k_scan_sums, dim3(scan_blocks), dim3(1024), 0, st, P.deg, nodes, scan_per, scan_part);
+    hipLaunchKernelGGL(k_scan, dim3(scan_blocks), dim3(1024), 0, st, P.deg, nodes, scan_per, scan_part, P.off);
     HM_LAUNCH_CHECK("k_scan");
     size_t tmp_bytes = P.sort_tmp_bytes;
     HM_HIP(hipcub::DeviceRadixSort::SortPairs(P.sort_tmp, tmp_bytes, P.keys_in, P.keys_out, P.vals_in, P.eid,
