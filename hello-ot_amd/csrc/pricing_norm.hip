@@ -257,9 +257,10 @@ inline unsigned prep_blocks(int64_t n) {
 }
 
 // the fp32 entry threshold of a column whose running k-th value is kth: any pair whose fp32 score is at or below
-// it has an exact score below kth (one ulp down keeps it strictly below kth - slack)
+// it has an exact score below kth (one ulp down keeps it strictly below kth - slack). A slack that is not finite (a dual
+// that is infinite, or whose slack is beyond fp32) leaves none: inf - inf would be a threshold that nothing passes.
 __device__ inline float column_threshold(double kth, float cslack) {
-    return (kth == -INFINITY) ? -INFINITY : nextafterf((float)(kth - (double)cslack), -INFINITY);
+    return (kth == -INFINITY || !(cslack < INFINITY)) ? -INFINITY : nextafterf((float)(kth - (double)cslack), -INFINITY);
 }
 
 // marks the unused slots of the wave's run empty (every lane of the wave calls it)
@@ -396,7 +397,7 @@ __global__ __launch_bounds__(256) void norm_seed(const float* __restrict__ X, Sw
 
 // The threshold a row's seeds give: fp32 scores at or below it belong to pairs whose exact score is below the row's k-th
 // best. A seed is within slack of an exact score (l2: within 1.5 of them, its square root being off by one unit in the
-// last place), and a pair's fp32 score within slack of its exact one.
+// last place), and a pair's fp32 score within slack of its exact one. None for a slack that is not finite (column_threshold).
 __device__ __forceinline__ float seed_threshold(const unsigned int* __restrict__ seeds, int64_t m, int64_t row, int k,
                                                 float slack) {
     unsigned int lo = 0xffffffffu;
@@ -405,7 +406,7 @@ __device__ __forceinline__ float seed_threshold(const unsigned int* __restrict__
         lo = s < lo ? s : lo;
     }
     const float v = key_float(lo);
-    return v > -INFINITY ? nextafterf((float)((double)v - 2.5 * (double)slack), -INFINITY) : -INFINITY;
+    return v > -INFINITY && slack < INFINITY ? nextafterf((float)((double)v - 2.5 * (double)slack), -INFINITY) : -INFINITY;
 }
 
 // Bound: fp32 VALU (two operations per feature and pair; l1 at d = 8: 16 of about 23 instructions per pair). So the
@@ -634,7 +635,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sweep_waves
                         }
                         sWorst[r * T] = at;
                         float thr = sThr[r * T];
-                        if (kth > -INFINITY) thr = fmaxf(thr, nextafterf((float)(kth - (double)slack), -INFINITY));
+                        thr = fmaxf(thr, column_threshold(kth, slack));
                         sThr[r * T] = thr;
                         const float lo = ST ? fminf(thr, -slack) : thr;
 #pragma unroll

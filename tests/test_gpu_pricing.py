@@ -562,6 +562,43 @@ def test_norm_sweep_widths_tiles_and_list_lengths(cuda, kind, m, n, d, k):
     _assert_stats(st, ost)
 
 
+@pytest.mark.parametrize("kind", [0, 1, 2])
+@pytest.mark.parametrize("k", [1, 2, 8])
+@pytest.mark.parametrize("d", [6, 150])
+@pytest.mark.parametrize("duals", ["f+", "f-", "g+", "g-", "f1e46", "g1e46", "-g1e46", "f+g+", "f+g-"])
+def test_norm_duals_without_a_finite_slack(cuda, kind, k, d, duals):
+    """An infinite dual, or one whose slack fp32 holds as infinity, leaves no threshold to filter by: lists, counts and
+    maximum are the oracle's, in the sweeps with both directions (k <= 2 with the column lists on the row sweep) and with
+    rows alone. (Pairs at -inf stay out of the lists; the oracle's fill them up.)"""
+    rng = np.random.default_rng(3 * k + d)
+    m, n = 520, 600
+    X = rng.random((m, d)).astype(np.float32)
+    Y = rng.random((n, d)).astype(np.float32)
+    f, g = rng.normal(0.5, 0.3, m) * d ** 0.5, rng.normal(0.5, 0.3, n) * d ** 0.5
+    sign = {"+": np.inf, "-": -np.inf}
+    if duals[-4:] == "1e46":
+        (f if duals[0] == "f" else g)[300] = -1e46 if duals[0] == "-" else 1e46
+    else:
+        for dual, s in zip(duals[::2], duals[1::2]):
+            (f if dual == "f" else g)[[510, 7]] = sign[s]
+    orv, ori, ocv, oci, ost = oracle.norm_scan(X, Y, f, g, k, kind)
+    ori, oci = np.where(np.isneginf(orv), -1, ori), np.where(np.isneginf(ocv), -1, oci)
+    if duals == "-g1e46":  # fp32 holds the column's scores as -inf
+        ocv[300], oci[300] = -np.inf, -1
+    t = _to(cuda, X, Y, f, g)
+    for cols in (True, False):
+        rv, ri, cv, ci, st = pricing_norm(*t, k, kind, cols=cols)
+        np.testing.assert_array_equal(rv.cpu().numpy(), orv)
+        np.testing.assert_array_equal(ri.cpu().numpy(), ori)
+        if cols:
+            np.testing.assert_array_equal(cv.cpu().numpy(), ocv)
+            np.testing.assert_array_equal(ci.cpu().numpy(), oci)
+        _assert_stats(st, ost)
+    rv, ri, _, _, _ = pricing_norm(*t, k, kind, cols=False, stats=False)
+    np.testing.assert_array_equal(rv.cpu().numpy(), orv)
+    np.testing.assert_array_equal(ri.cpu().numpy(), ori)
+
+
 @pytest.mark.parametrize("kind,d", [(0, 3), (1, 8), (2, 20), (0, 32)])
 def test_norm_two_rows_per_thread_agree_with_one(cuda, kind, d):
     """Large sides with short lists run two rows per thread and, with both directions, column lists on the row sweep;
