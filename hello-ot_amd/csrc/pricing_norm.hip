@@ -397,7 +397,9 @@ __global__ __launch_bounds__(256) void norm_seed(const float* __restrict__ X, Sw
 
 // The threshold a row's seeds give: fp32 scores at or below it belong to pairs whose exact score is below the row's k-th
 // best. A seed is within slack of an exact score (l2: within 1.5 of them, its square root being off by one unit in the
-// last place), and a pair's fp32 score within slack of its exact one. None for a slack that is not finite (column_threshold).
+// last place, and by up to 2^-63 where the instruction takes a denormal square for 0), and a pair's fp32 score within slack
+// of its exact one. None for a slack that is not finite (column_threshold).
+template <int KIND>
 __device__ __forceinline__ float seed_threshold(const unsigned int* __restrict__ seeds, int64_t m, int64_t row, int k,
                                                 float slack) {
     unsigned int lo = 0xffffffffu;
@@ -406,7 +408,8 @@ __device__ __forceinline__ float seed_threshold(const unsigned int* __restrict__
         lo = s < lo ? s : lo;
     }
     const float v = key_float(lo);
-    return v > -INFINITY && slack < INFINITY ? nextafterf((float)((double)v - 2.5 * (double)slack), -INFINITY) : -INFINITY;
+    const double off = 2.5 * (double)slack + (KIND == HM_COST_L2 ? 1.0842021724855044e-19 : 0.0);
+    return v > -INFINITY && slack < INFINITY ? nextafterf((float)((double)v - off), -INFINITY) : -INFINITY;
 }
 
 // Bound: fp32 VALU (two operations per feature and pair; l1 at d = 8: 16 of about 23 instructions per pair). So the
@@ -476,7 +479,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sweep_waves
         // slack >= |sigma32 - sigma64|: every fp32 operand is within u of its fp64 value and the two fp32 sums
         // round by at most u each; magnitudes are bounded by |g| + c + |f| with c <= ||x||_1 + max||y||_1.
         const float slack = (float)((x1 + ymax1 + gmax + fabs(fi)) * 4.0 * 5.9604644775390625e-08 * (1.0 + 1e-6) + 1e-37);
-        const float thr = ok && seeds ? seed_threshold(seeds, m, row, k, slack) : -INFINITY;
+        const float thr = ok && seeds ? seed_threshold<KIND>(seeds, m, row, k, slack) : -INFINITY;
         fi32[r] = ok ? (float)fi : -INFINITY;
         low[r] = ST ? fminf(thr, -slack) : thr;
         sF[r * T] = fi;
@@ -535,7 +538,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sweep_waves
             c.thr = INFINITY;
             if constexpr (FUSED) {
                 c.thr = column_threshold(running_kth(ca, t0 + e, k), cslack);
-                if (ca.seeds) c.thr = fmaxf(c.thr, seed_threshold(ca.seeds, ca.n, t0 + e, k, cslack));
+                if (ca.seeds) c.thr = fmaxf(c.thr, seed_threshold<KIND>(ca.seeds, ca.n, t0 + e, k, cslack));
             }
             sG[e] = c;
         }

@@ -599,6 +599,26 @@ def test_norm_duals_without_a_finite_slack(cuda, kind, k, d, duals):
     np.testing.assert_array_equal(ri.cpu().numpy(), ori)
 
 
+@pytest.mark.parametrize("kind", [0, 1, 2])
+@pytest.mark.parametrize("scale", [1e-18, 1e-20, 3e-23])
+def test_norm_lists_of_tiny_costs(cuda, kind, scale):
+    """Costs whose squares are fp32 denormals, or 0: the entry floors, the squared test of the l2 sweep and the lists keep
+    what the oracle keeps."""
+    rng = np.random.default_rng(17)
+    m, n, d = 300, 2100, 6
+    X = (scale * rng.random((m, d))).astype(np.float32)
+    Y = (scale * rng.random((n, d))).astype(np.float32)
+    f, g = scale * rng.normal(0.3, 0.2, m), scale * rng.normal(0.3, 0.2, n)
+    for k in (1, 2, 8):
+        orv, ori, ocv, oci, ost = oracle.norm_scan(X, Y, f, g, k, kind)
+        rv, ri, cv, ci, st = pricing_norm(*_to(cuda, X, Y, f, g), k, kind)
+        np.testing.assert_array_equal(ri.cpu().numpy(), ori)
+        np.testing.assert_array_equal(rv.cpu().numpy(), orv)
+        np.testing.assert_array_equal(ci.cpu().numpy(), oci)
+        np.testing.assert_array_equal(cv.cpu().numpy(), ocv)
+        assert int(st[2]) == ost[2] and float(st[3]) == ost[3]
+
+
 @pytest.mark.parametrize("kind,d", [(0, 3), (1, 8), (2, 20), (0, 32)])
 def test_norm_two_rows_per_thread_agree_with_one(cuda, kind, d):
     """Large sides with short lists run two rows per thread and, with both directions, column lists on the row sweep;
