@@ -10,8 +10,8 @@
 // One thread owns one or two X rows (features in registers up to d = 128); a Y row is the same for the whole wave, so
 // its features are scalar loads and enter the vector instructions as scalar operands. Per pair the loop computes the
 // cost and one test against the lowest of the row's, the column's and the certificate's thresholds; what passes (a few
-// pairs in a thousand) is handled out of line, with the row lists in LDS. Certificate sums are accumulated in fp32 per
-// tile and flushed to fp64.
+// pairs in a thousand) is handled out of line, with the row lists in LDS. The certificate adds the squares of violated
+// scores in fp64 and those of all costs in fp32, flushed to fp64 per tile or more often (cost_span).
 //
 // Column lists, k <= 2 with rows and columns requested: they ride on the row sweep, so every pair is evaluated
 // once. Every column keeps its running top-2 values in global memory (the largest and second largest score
@@ -359,6 +359,11 @@ constexpr int sweep_waves(int dr, int r) {
     return dr == 0 ? 3 : dr * r <= 32 ? 5 : dr * r <= 64 ? 4 : 3;
 }
 
+// squared costs added up in fp32 before they go to the fp64 sum (0: each goes there): a chain of L rounds by up to L / 2
+// units of 2^-24. A tile where a pair is cheap; 32 for wider rows, where the flush is lost in the pairs' work (as is one
+// fp64 operation a pair for streamed rows).
+constexpr int cost_span(int dr) { return dr == 0 ? 0 : dr <= 48 ? NT : 32; }
+
 // Entry floors of the row lists, before the sweep: the k-th best score of a row is at least the smallest of k maxima over
 // disjoint samples of its columns. Sample q of `samples` (grid y) takes every samples-th of `count` columns spread over
 // the side and raises seeds[(q % k) * m + row] (an ordered key) to its largest fp32 score. Without floors every segment
@@ -545,121 +550,131 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sweep_waves
         if (tid < J - 1) sG[cnt + tid] = TileCol{-INFINITY, INFINITY};  // columns past the tile never pass a test
         __syncthreads();
         const float* const yt = t0 >= side.tail_row ? side.tail + (t0 - side.tail_row) * d : side.Y + t0 * d;
-        float tden[R];
+        constexpr int SPAN = ST && cost_span(DR) > 0 ? cost_span(DR) : NT;
+        for (int j0 = 0; j0 < (SPAN < NT ? cnt : 1); j0 += SPAN) {
+            const int j1 = SPAN < NT && cnt > j0 + SPAN ? j0 + SPAN : cnt;
+            std::conditional_t<cost_span(DR) == 0, double, float> tden[R];
 #pragma unroll
-        for (int r = 0; r < R; ++r) tden[r] = 0.0f;
-        for (int jj = 0; jj < cnt; jj += J) {
-            // columns jj .. jj + J - 1 of the tile (past its end: the last one again)
-            ScalarRow y[J];
+            for (int r = 0; r < R; ++r) tden[r] = 0;
+            for (int jj = j0; jj < j1; jj += J) {
+                // columns jj .. jj + J - 1 of the tile (past its end: the last one again)
+                ScalarRow y[J];
 #pragma unroll
-            for (int u = 0; u < J; ++u) y[u] = scalar_row(yt + (unsigned)((jj + u < cnt ? jj + u : cnt - 1) * d));
-            TileCol col[J];
+                for (int u = 0; u < J; ++u) y[u] = scalar_row(yt + (unsigned)((jj + u < cnt ? jj + u : cnt - 1) * d));
+                TileCol col[J];
 #pragma unroll
-            for (int u = 0; u < J; ++u) col[u] = sG[jj + u];
-            float acc[J][R];
-            if constexpr (DR > 0) accumulate_reg<KIND, DR, R, J, TAIL>(x, y, d, acc);
-            else accumulate_mem<KIND, J>(X + (row0 < m ? row0 : 0) * d, y, d, acc);  // lanes past m read row 0
-            unsigned long long hits = 0ull;
+                for (int u = 0; u < J; ++u) col[u] = sG[jj + u];
+                float acc[J][R];
+                if constexpr (DR > 0) accumulate_reg<KIND, DR, R, J, TAIL>(x, y, d, acc);
+                else accumulate_mem<KIND, J>(X + (row0 < m ? row0 : 0) * d, y, d, acc);  // lanes past m read row 0
+                unsigned long long hits = 0ull;
 #pragma unroll
-            for (int u = 0; u < J; ++u) {
+                for (int u = 0; u < J; ++u) {
 #pragma unroll
-                for (int r = 0; r < R; ++r) {
-                    if constexpr (KIND == HM_COST_L2) {
-                        const float t = FUSED ? fminf(low[r], col[u].thr) : low[r];
-                        const float b = (col[u].g + fi32[r]) - t;
-                        hits |= __ballot(acc[u][r] <= b * fabsf(b));
-                    } else {
-                        const float sc = (col[u].g - acc[u][r]) + fi32[r];
-                        hits |= __ballot(sc > low[r]);
-                        if (FUSED) hits |= __ballot(sc > col[u].thr);
-                    }
-                    if (ST) cm[r] = fmaxf(cm[r], acc[u][r]);  // (a column past the tile repeats its last one)
-                }
-                if (ST) {
-                    if (u == 0 || jj + u < cnt) {
-                        asm volatile("");  // a scalar branch, not a select per accumulator
-#pragma unroll
-                        for (int r = 0; r < R; ++r)
-                            tden[r] = KIND == HM_COST_L2 ? tden[r] + acc[u][r] : fmaf(acc[u][r], acc[u][r], tden[r]);
-                    }
-                }
-            }
-            if (!hits) continue;
-            // rare: some lane has a pair that may matter; each pair of the step in turn
-#pragma unroll 1
-            for (int e = 0; e < J * R; ++e) {
-                float a = acc[0][0], f32 = fi32[0];
-#pragma unroll
-                for (int u = 0; u < J; ++u)
-#pragma unroll
-                    for (int r = 0; r < R; ++r)
-                        if (e == u * R + r) {
-                            a = acc[u][r];
-                            f32 = fi32[r];
+                    for (int r = 0; r < R; ++r) {
+                        if constexpr (KIND == HM_COST_L2) {
+                            const float t = FUSED ? fminf(low[r], col[u].thr) : low[r];
+                            const float b = (col[u].g + fi32[r]) - t;
+                            hits |= __ballot(acc[u][r] <= b * fabsf(b));
+                        } else {
+                            const float sc = (col[u].g - acc[u][r]) + fi32[r];
+                            hits |= __ballot(sc > low[r]);
+                            if (FUSED) hits |= __ballot(sc > col[u].thr);
                         }
-                const int u = e / R, r = e % R;
-                const float gj32 = sG[jj + u].g;
-                const int64_t j = t0 + jj + u;
-                const float c = cost_of<KIND>(a);
-                const float s32 = (gj32 - c) + f32;
-                if constexpr (FUSED) {
-                    const bool over = s32 > sG[jj + u].thr;
-                    if (__any(over)) {
-                        const double sig = (cb[j] - (double)c) + sF[r * T];
-                        column_enter(ca, run, over && sig == sig, j, sig, (int)(row0 + (int64_t)r * T), k, sOwn + jj + u,
-                                     sOwn + NT + jj + u, &sG[jj + u].thr, cslack);
+                        if (ST) cm[r] = fmaxf(cm[r], acc[u][r]);  // (a column past the tile repeats its last one)
                     }
-                }
-                const bool enters = s32 > sThr[r * T];
-                const float slack = sSlack[r * T];
-                const bool near = ST && s32 > -slack;
-                if (enters || near) {
-                    const double cd = (double)c, fi = sF[r * T], gj = cb[j];
-                    const double sig = TRANSPOSED ? (fi - cd) + gj : (gj - cd) + fi;
-                    double* const v = sV + (size_t)r * k * T;
-                    int* const id = sI + (size_t)r * k * T;
-                    const int w = sWorst[r * T];
-                    if (enters && sig == sig && better(sig, (int)j, v[w * T], id[w * T])) {
-                        // the list is unordered: the new entry replaces the worst, and the worst of the rest is found by
-                        // independent reads (a sorted insertion is a chain of dependent ones)
-                        v[w * T] = sig;
-                        id[w * T] = (int)j;
-                        double kth = v[0];
-                        int kid = id[0], at = 0;
-#pragma unroll 4
-                        for (int s = 1; s < k; ++s) {
-                            const double vs = v[s * T];
-                            const int is = id[s * T];
-                            if (better(kth, kid, vs, is)) {
-                                kth = vs;
-                                kid = is;
-                                at = s;
+                    if (ST) {
+                        if (u == 0 || jj + u < cnt) {
+                            asm volatile("");  // a scalar branch, not a select per accumulator
+#pragma unroll
+                            for (int r = 0; r < R; ++r) {
+                                if constexpr (cost_span(DR) == 0) {
+                                    const double c = acc[u][r];
+                                    tden[r] = KIND == HM_COST_L2 ? tden[r] + c : fma(c, c, tden[r]);
+                                } else {
+                                    tden[r] = KIND == HM_COST_L2 ? tden[r] + acc[u][r] : fmaf(acc[u][r], acc[u][r], tden[r]);
+                                }
                             }
                         }
-                        sWorst[r * T] = at;
-                        float thr = sThr[r * T];
-                        thr = fmaxf(thr, column_threshold(kth, slack));
-                        sThr[r * T] = thr;
-                        const float lo = ST ? fminf(thr, -slack) : thr;
-#pragma unroll
-                        for (int q = 0; q < R; ++q)
-                            if (q == r) low[q] = lo;
                     }
-                    // beyond the slack the fp32 score decides; within it the exact fp64 score does (the maximum
-                    // comes from the exact row lists afterwards)
-                    if (ST && s32 > slack) {
-                        num64 = fma((double)s32, (double)s32, num64);
-                        ++count;
-                    } else if (near && sig > 0.0) {
-                        num64 = fma(sig, sig, num64);
-                        ++count;
+                }
+                if (!hits) continue;
+                // rare: some lane has a pair that may matter; each pair of the step in turn
+#pragma unroll 1
+                for (int e = 0; e < J * R; ++e) {
+                    float a = acc[0][0], f32 = fi32[0];
+#pragma unroll
+                    for (int u = 0; u < J; ++u)
+#pragma unroll
+                        for (int r = 0; r < R; ++r)
+                            if (e == u * R + r) {
+                                a = acc[u][r];
+                                f32 = fi32[r];
+                            }
+                    const int u = e / R, r = e % R;
+                    const float gj32 = sG[jj + u].g;
+                    const int64_t j = t0 + jj + u;
+                    const float c = cost_of<KIND>(a);
+                    const float s32 = (gj32 - c) + f32;
+                    if constexpr (FUSED) {
+                        const bool over = s32 > sG[jj + u].thr;
+                        if (__any(over)) {
+                            const double sig = (cb[j] - (double)c) + sF[r * T];
+                            column_enter(ca, run, over && sig == sig, j, sig, (int)(row0 + (int64_t)r * T), k, sOwn + jj + u,
+                                         sOwn + NT + jj + u, &sG[jj + u].thr, cslack);
+                        }
+                    }
+                    const bool enters = s32 > sThr[r * T];
+                    const float slack = sSlack[r * T];
+                    const bool near = ST && s32 > -slack;
+                    if (enters || near) {
+                        const double cd = (double)c, fi = sF[r * T], gj = cb[j];
+                        const double sig = TRANSPOSED ? (fi - cd) + gj : (gj - cd) + fi;
+                        double* const v = sV + (size_t)r * k * T;
+                        int* const id = sI + (size_t)r * k * T;
+                        const int w = sWorst[r * T];
+                        if (enters && sig == sig && better(sig, (int)j, v[w * T], id[w * T])) {
+                            // the list is unordered: the new entry replaces the worst, and the worst of the rest is found by
+                            // independent reads (a sorted insertion is a chain of dependent ones)
+                            v[w * T] = sig;
+                            id[w * T] = (int)j;
+                            double kth = v[0];
+                            int kid = id[0], at = 0;
+#pragma unroll 4
+                            for (int s = 1; s < k; ++s) {
+                                const double vs = v[s * T];
+                                const int is = id[s * T];
+                                if (better(kth, kid, vs, is)) {
+                                    kth = vs;
+                                    kid = is;
+                                    at = s;
+                                }
+                            }
+                            sWorst[r * T] = at;
+                            float thr = sThr[r * T];
+                            thr = fmaxf(thr, column_threshold(kth, slack));
+                            sThr[r * T] = thr;
+                            const float lo = ST ? fminf(thr, -slack) : thr;
+#pragma unroll
+                            for (int q = 0; q < R; ++q)
+                                if (q == r) low[q] = lo;
+                        }
+                        // beyond the slack the fp32 score decides; within it the exact fp64 score does (the maximum
+                        // comes from the exact row lists afterwards)
+                        if (ST && s32 > slack) {
+                            num64 = fma((double)s32, (double)s32, num64);
+                            ++count;
+                        } else if (near && sig > 0.0) {
+                            num64 = fma(sig, sig, num64);
+                            ++count;
+                        }
                     }
                 }
             }
-        }
-        if (ST) {
+            if (ST) {
 #pragma unroll
-            for (int r = 0; r < R; ++r) den64[r] += (double)tden[r];
+                for (int r = 0; r < R; ++r) den64[r] += (double)tden[r];
+            }
         }
     }
     if constexpr (FUSED) {

@@ -600,6 +600,23 @@ def test_norm_duals_without_a_finite_slack(cuda, kind, k, d, duals):
 
 
 @pytest.mark.parametrize("kind", [0, 1, 2])
+@pytest.mark.parametrize("d,chain", [(64, 32), (100, 32), (128, 32), (129, 1), (1000, 1)])
+def test_norm_certificate_sums_of_wide_rows(cuda, kind, d, chain):
+    """Sum of squared costs with every cost the same: an fp32 chain then rounds in one direction. Rows of more than 48
+    features add up at most 32 squares in fp32 (relative error at most (32 + 1) / 2 units of 2^-24; this cost: 3.7e-6
+    over 256 of them), streamed rows none (l2: the square itself is an fp32 sum, one unit)."""
+    m, n, c = 40, 1100, np.float32(1.0519750118255615)
+    X = np.zeros((m, d), np.float32)
+    Y = np.zeros((n, d), np.float32)
+    Y[:, d // 2] = c
+    st = pricing_norm(*_to(cuda, X, Y, np.zeros(m), np.zeros(n)), 2, kind)[4]
+    want = m * n * float(c) ** 2
+    unit = 2.0 ** -24
+    bound = (0.5 * (chain + 1) if chain > 1 else 0.0) * unit + (unit if kind == 2 else 0.0) + 1e-12
+    assert abs(float(st[1]) / want - 1.0) <= bound
+
+
+@pytest.mark.parametrize("kind", [0, 1, 2])
 @pytest.mark.parametrize("scale", [1e-18, 1e-20, 3e-23])
 def test_norm_lists_of_tiny_costs(cuda, kind, scale):
     """Costs whose squares are fp32 denormals, or 0: the entry floors, the squared test of the l2 sweep and the lists keep
