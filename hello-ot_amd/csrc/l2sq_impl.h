@@ -545,8 +545,8 @@ __device__ __forceinline__ void sweep_row_init(SweepRow<K1>& s, int64_t row, int
 // 128 X rows, CPASS Y rows at a time (sC holds CPASS * CST floats; 256 / CPASS threads scan each row and merge
 // their lists). Ends with a barrier, so that the next tile may rewrite sDB / sGE / sC.
 // LANES (with FULL, without columns; l2sq_sweep_short, l2sq_sweep_split) takes ragged tiles and panels without a per-pair test: Y rows
-// beyond the segment have the bias -inf, which no list, vote or decision lets through (only the cost sums test the
-// limit, in ragged tiles), the caller drops the sums of lanes beyond the panel, and has its own barrier per tile. A second
+// beyond the segment have the bias -inf in sDB and sDB64, which no list or decision lets through (only the cost sums test
+// the limit, in ragged tiles), the caller drops the sums of lanes beyond the panel, and has its own barrier per tile. A second
 // copy for ragged tiles made the compiler keep its 64 limit tests and spill 150 to 400 vectors a lane: 60001 x 60001, d = 4,
 // with the certificate 9.4 ms with it, 4.3 without; 65536 x 131072, d = 64 (split copies) 8.3 and 7.1.
 template <int K1, bool COLS, bool APPEND, int CPASS, bool FULL, bool ST, bool SRT = false, bool LANES = false>
@@ -684,8 +684,9 @@ __device__ __forceinline__ void sweep_epilogue(const v16f (&tot)[NB], SweepRow<K
             for (int q = 0; q < 16; ++q) {
                 const int jl = b * 32 + 8 * (q / 4) + 4 * h + (q % 4);
                 const float t = tot[b][q];
-                // (LANES: an infinite slack, from a dual beyond fp32, would let the columns past the segment through)
-                const bool in = LANES ? sDB[jl] > -INFINITY : FULL || 4 * h < ylim - (jl - 4 * h);
+                // (LANES: an infinite slack, from a dual beyond fp32, lets the columns past the segment through, whose fp64
+                // bias of -inf is never a positive score)
+                const bool in = FULL || 4 * h < ylim - (jl - 4 * h);
                 cert_near(rok && in, t, fmaf(scale, t, sDB[jl]), s.qbi, slack, scale, qb64, sDB64[jl], tcnt, s.num64);
             }
         }
@@ -1074,7 +1075,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void l
             gdb = j < y_end ? db32[j] : -INFINITY;
             if (ST) {
                 gge = (STATS && j < y_end) ? ge32[j] : 0.0f;
-                gdb64 = (STATS && j < y_end) ? cert.db[j] : 0.0;
+                gdb64 = (STATS && j < y_end) ? cert.db[j] : -INFINITY;
             }
         }
     };
@@ -1457,8 +1458,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(COLS ? 1 : 
             step(I3{});
         }
         if constexpr (!COLS && !APPEND) {
-            if (y_end - ytile < (int64_t)BY) {  // (LANES: the bias of the columns past the segment)
-                if (tid < BY && ytile + tid >= y_end) sDB[tid] = -INFINITY;
+            if (y_end - ytile < (int64_t)BY) {  // (LANES: the biases of the columns past the segment)
+                if (tid < BY && ytile + tid >= y_end) {
+                    sDB[tid] = -INFINITY;
+                    if (stats) sDB64[tid] = -INFINITY;
+                }
                 __syncthreads();
             }
             sweep_epilogue<K1, false, false, BY, true, ST, true, true>(

@@ -182,6 +182,21 @@ def test_l2sq_count_with_a_dual_beyond_fp32(cuda, d, precision):
     assert (sigma > near).sum() <= int(st[2]) <= (sigma > -near).sum()
 
 
+@pytest.mark.parametrize("d,precision", [(1, "fp32"), (40, "fp32"), (5, "bf16x3"), (100, "bf16x3")])
+def test_l2sq_count_with_a_column_bias_that_fp32_holds_as_infinite(cuda, d, precision):
+    """A violated pair whose column bias is -inf in fp32 and finite in fp64: under an infinite slack (the other columns'
+    biases) its sign is taken in fp64, and it counts."""
+    m, n = 130, 300
+    X, Y = np.zeros((m, d), np.float32), np.zeros((n, d), np.float32)
+    qb, db = np.zeros(m), np.full(n, -1e50)
+    X[3, 0] = Y[7, 0] = 2.0 ** 53                       # scale 1: their score is 2^106 - 1e29
+    qb[3], db[7] = 3.402823567e38, -3.402823568e38
+    st = pricing_l2sq(*_to(cuda, X, Y, np.zeros(m), np.zeros(n), qb, db), 1, dot_scale=1.0, rows=False, cols=False,
+                      stats=True, precision=precision)[4]
+    assert int(st[2]) == 1
+    np.testing.assert_allclose(float(st[0]), (2.0 ** 106 + qb[3] + db[7]) ** 2, rtol=1e-6)
+
+
 @pytest.mark.parametrize("side", ["x", "y"])
 @pytest.mark.parametrize("d", [5, 256])
 @pytest.mark.parametrize("precision", ["fp32", "bf16x3", "int8x3"])
