@@ -29,6 +29,7 @@
 // association).
 #include <hipcub/hipcub.hpp>
 
+#include <algorithm>
 #include <mutex>
 #include <type_traits>
 
@@ -1039,6 +1040,12 @@ inline size_t scan_tmp_bytes(int64_t n) {
     return bytes;
 }
 
+// certificate partials: of the row sweep, which in a fused call takes them in any case
+inline size_t blockstats_doubles(const NormPlan& rows, int64_t m, uint32_t flags, int64_t cap) {
+    const int64_t per = (int64_t)rows.R * rows.T;
+    return (flags & HM_STATS) || cap > 0 ? (size_t)5 * ((m + per - 1) / per) * rows.S : 1;
+}
+
 // cap > 0: the fused path with a candidate buffer of cap entries
 template <class A>
 void norm_layout(A& a, int64_t m, int64_t n, int d, int k, uint32_t flags, bool seeded, int64_t cap, NormWork& w) {
@@ -1051,8 +1058,7 @@ void norm_layout(A& a, int64_t m, int64_t n, int d, int k, uint32_t flags, bool 
     }
     w.pv = a.template take<double>(entries > 0 ? entries : 1);
     w.pi = a.template take<int>(entries > 0 ? entries : 1);
-    const int64_t br = ((m + pr.R * pr.T - 1) / (pr.R * pr.T)) * pr.S, bc = ((n + pc.R * pc.T - 1) / (pc.R * pc.T)) * pc.S;
-    w.bs = a.template take<double>((size_t)5 * (br > bc ? br : bc));
+    w.bs = a.template take<double>(blockstats_doubles(pr, m, flags, cap));
     w.maxima = a.template take<unsigned long long>(5);
     const bool fp32 = !(flags & HM_FP64);
     w.ytail = a.template take<float>(fp32 && (flags & (HM_ROWS | HM_STATS)) ? tail_floats(n, d) : 1);
@@ -1412,9 +1418,16 @@ int norm_scan_run(void* stream, const float* X, const float* Y, const double* f,
 // Scratch of the allocation-free entry point: one array per GPU, for the life of the process. Host code reaches it
 // only through the device address hipGetSymbolAddress returns (looked up once per device, under a lock).
 constexpr size_t NORM_SCRATCH_BYTES = size_t(64) << 20;
-// room beyond them for the padded copies of the sides' last rows, which grow with d alone, and their alignment
-constexpr size_t NORM_TAIL_BYTES = size_t(2) * (2 * NT * REG_FEATURES + PAD) * sizeof(float) + 1024;
-__device__ __align__(256) unsigned char scratch[NORM_SCRATCH_BYTES + NORM_TAIL_BYTES];
+// The lists get all of them: beyond them there is room for the padded copies of the sides' last rows, which grow with d
+// alone, for the certificate partials (40 bytes a workgroup of 256 rows or 128, whose lists take at least 12 k each, k > 16
+// for 128: at most 5/384 of the lists' bytes, and one workgroup more for each of 64 segments), and for alignment.
+constexpr size_t NORM_ROOM_BYTES = size_t(2) * (2 * NT * REG_FEATURES + PAD) * sizeof(float) +
+                                   NORM_SCRATCH_BYTES / 384 * 5 + 64 * 40 + 2048;
+__device__ __align__(256) unsigned char scratch[NORM_SCRATCH_BYTES + NORM_ROOM_BYTES];
+inline size_t noalloc_room(int64_t m, int64_t n, int d, int k, uint32_t flags) {
+    return (tail_floats(n, d) + tail_floats(m, d)) * sizeof(float) +
+           blockstats_doubles(norm_plan(m, n, d, k, flags), m, flags, 0) * sizeof(double) + 2048;
+}
 constexpr int SCRATCH_DEVICES = 64;
 std::mutex scratch_lock;
 void* scratch_address[SCRATCH_DEVICES] = {};
@@ -1453,9 +1466,9 @@ extern "C" int hm_pricing_norm_noalloc(void* stream, const float* X, const float
     HM_CHECK_ARG(m >= 1 && n >= 1 && k >= 1 && k <= 32, "norm pricing requires nonempty inputs and 1 <= k <= 32");
     if (int rc = check_features(d, flags)) return rc;
     // the two-sweep path's scratch; the fused path runs when its larger scratch fits as well
-    const size_t room = (tail_floats(n, d) + tail_floats(m, d)) * sizeof(float) + 1024;
+    const size_t bytes = NORM_SCRATCH_BYTES + std::min(noalloc_room(m, n, d, k, flags), NORM_ROOM_BYTES);
     const size_t need = norm_workspace(m, n, d, k, flags, false, 0);
-    if (need > NORM_SCRATCH_BYTES + room)
+    if (need > bytes)
         return fail(HM_ENOSPC, "norm pricing (no-alloc): this call needs %zu bytes of scratch, above the %zu-byte static "
                                "scratch array; call hm_pricing_norm with a workspace instead",
                     need, NORM_SCRATCH_BYTES);
@@ -1464,5 +1477,5 @@ extern "C" int hm_pricing_norm_noalloc(void* stream, const float* X, const float
     const ProfileOff no_events;  // timing events would be created on demand
     // the fused path only with its full candidate buffer: a partial one that overflows would cost both sweeps
     return norm_scan_run(stream, X, Y, f, g, m, n, d, k, kind, flags, row_val, row_idx, col_val, col_idx, stats,
-                         scratch_ptr, NORM_SCRATCH_BYTES + room, false);
+                         scratch_ptr, bytes, false);
 }

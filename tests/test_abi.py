@@ -60,6 +60,26 @@ def test_workspace_queries_are_host_arithmetic():
     assert lib.hm_pricing_norm_workspace_bytes(524288, 524288, 8, 2, 7) > 0
 
 
+@pytest.mark.parametrize("m,n,d,k,flags", [
+    (232888, 4, 545, 24, 3),            # rows and columns, lists of more than 16: workgroups of 128 rows
+    (328711, 17, 135, 17, 15),          # the same with the certificate
+    (174690, 195, 1, 32, 3),            # padded copies of short rows
+    (382898944, 395, 4, 24, 2),         # columns alone, a tall other side
+    (5592405, 1, 1, 1, 7),              # one list entry a row: as many workgroups as the lists allow
+])
+def test_noalloc_norm_scan_takes_lists_of_64_mib(m, n, d, k, flags):
+    """The static scratch of hm_pricing_norm_noalloc holds 64 MiB of lists and beside them what grows with the call's other
+    sizes: calls at that limit are not refused for space (the null inputs are, or the missing device); a list more is."""
+    lib = _lib.load()
+    for rows, fits in ((m, True), (m + (m >> 8) + (1 << 16), False)):
+        rc = lib.hm_pricing_norm_noalloc(None, None, None, None, None, rows, n, d, k, 0, flags, None, None, None, None, None)
+        assert rc != _lib.HM_OK
+        if flags != 2:                  # (columns alone: the lists are the columns')
+            assert ("bytes of scratch" in _lib.last_error()) != fits
+        elif fits:
+            assert "bytes of scratch" not in _lib.last_error()
+
+
 def test_resident_side_sizes_and_validation():
     """A resident Y side holds its norms and sweep copy (two bytes per feature for the int8 split, four for
     split-bf16, none for fp32); a call against it needs that much less workspace. Invalid calls fail before any
