@@ -752,15 +752,17 @@ struct SidePlan {
 
 constexpr int GL = 8;  // lanes per group
 
-// One PDHG iteration: workgroups [0, src.blocks) run the source side, the rest the target side. Small problems are
-// bound by the latency of a launch and of each pass's chain of dependent loads (offsets, edges, gathered dual, fold),
-// which the two sides now share: 4096 nodes a side and 61 thousand edges take 10.0 us an iteration, as two dependent
-// launches they took 11.3. Large ones stream the edge state (524288 a side, 12.5 million edges: 318 us, before 324).
+// One PDHG iteration: workgroups [0, src.blocks) run the source side, the rest the target side (the first `first` of them
+// in earlier launches). Small problems are bound by the latency of a launch and of each pass's chain of dependent loads
+// (offsets, edges, gathered dual, fold), which the two sides now share: 4096 nodes a side and 61 thousand edges take 10.0 us
+// an iteration, as two dependent launches they took 11.3. Large ones stream the edge state (524288 a side, 12.5 million
+// edges: 318 us, before 324).
 template <bool CHECKPOINT, bool STORE>
-__global__ __launch_bounds__(PT) void k_iteration(const Pdhg P, SidePlan src, SidePlan tgt, const double* __restrict__ cur,
-                                                  double* __restrict__ next, double ps, double ds, double h) {
+__global__ __launch_bounds__(PT) void k_iteration(const Pdhg P, SidePlan src, SidePlan tgt, int64_t first,
+                                                  const double* __restrict__ cur, double* __restrict__ next, double ps,
+                                                  double ds, double h) {
     __shared__ BlockLds lds;
-    const int64_t b = blockIdx.x;
+    const int64_t b = first + blockIdx.x;
     if (b < src.blocks) {
         const Side sd{0, P.n, P.n, 0, P.col, P.cs, P.ax, P.x, P.px, P.dx, P.loc_s, P.g16_s, P.gbase_s};
         if (src.u == 0) block_pass<true, CHECKPOINT, STORE>(P, sd, b, src.npb, cur, next, ps, ds, h, lds);
@@ -1068,10 +1070,18 @@ inline SidePlan side_plan(int64_t e, int64_t nodes, int max_degree) {
 // read only by the evaluation that follows one.
 int launch_iteration(hipStream_t st, const Pdhg& P, const SidePlan& src, const SidePlan& tgt, const double* cur,
                      double* next, bool checkpoint, bool major, double ps, double ds, double h) {
-    const dim3 grid((unsigned)(src.blocks + tgt.blocks)), block(PT);
-    if (major) hipLaunchKernelGGL((k_iteration<true, true>), grid, block, 0, st, P, src, tgt, cur, next, ps, ds, h);
-    else if (checkpoint) hipLaunchKernelGGL((k_iteration<true, false>), grid, block, 0, st, P, src, tgt, cur, next, ps, ds, h);
-    else hipLaunchKernelGGL((k_iteration<false, false>), grid, block, 0, st, P, src, tgt, cur, next, ps, ds, h);
+    // (a launch of 2^32 threads or more runs some of them; the lane groups take 8 a node)
+    constexpr int64_t MOST = (int64_t)UINT32_MAX / PT;
+    const int64_t blocks = src.blocks + tgt.blocks;
+    for (int64_t first = 0; first < blocks; first += MOST) {
+        const dim3 grid((unsigned)(blocks - first < MOST ? blocks - first : MOST)), block(PT);
+        if (major)
+            hipLaunchKernelGGL((k_iteration<true, true>), grid, block, 0, st, P, src, tgt, first, cur, next, ps, ds, h);
+        else if (checkpoint)
+            hipLaunchKernelGGL((k_iteration<true, false>), grid, block, 0, st, P, src, tgt, first, cur, next, ps, ds, h);
+        else
+            hipLaunchKernelGGL((k_iteration<false, false>), grid, block, 0, st, P, src, tgt, first, cur, next, ps, ds, h);
+    }
     HM_LAUNCH_CHECK("pdhg iteration");
     return HM_OK;
 }

@@ -450,6 +450,33 @@ def test_pdhg_resident_runs_match_oracle(cuda, ns, nt, per_row, hub, freq, check
     np.testing.assert_allclose(r.y.cpu().numpy(), ref["y"], rtol=1e-9, atol=1e-12)
 
 
+def test_pdhg_more_nodes_than_one_launch_of_both_sides_takes(cuda, monkeypatch):
+    """A small LP among 2^29 + 2000 nodes without mass or edges: an iteration's workgroups of both sides (8 threads a node)
+    are more than a launch takes. The extra nodes stay at 0 and leave every other node's and edge's operations as they
+    are; the small LP alone differs by the orders of the norm sums, which set the primal weight."""
+    monkeypatch.setenv("HELLOOT_PDHG_REORDER", "off")
+    ns, nt, more = 60, 45, (1 << 28) + 1000
+    rows, cols, costs, a, b = _sparse_lp(4, ns, nt, 240)
+    keep = np.zeros(rows.size, bool)                     # at most 8 edges a node: lane groups
+    deg = np.zeros(ns + nt, int)
+    for k, (i, j) in enumerate(zip(rows, cols)):
+        if deg[i] < 8 and deg[ns + j] < 8:
+            keep[k] = True
+            deg[[i, ns + j]] += 1
+    rows, cols, costs = rows[keep], cols[keep], costs[keep]
+    pad = lambda v: torch.cat((torch.as_tensor(v, device=cuda), torch.zeros(more - v.size, dtype=torch.float64, device=cuda)))
+    lp = NativeRestrictedOTPDLP(device=cuda, evaluation_frequency=10, iteration_limit=40)
+    ref = lp.solve_restricted(rows=rows, cols=cols, costs=costs, source_mass=a, target_mass=b, tolerance=0.0)
+    r = lp.solve_restricted(rows=rows, cols=cols, costs=costs, source_mass=pad(a), target_mass=pad(b), tolerance=0.0)
+    assert r.iterations == ref.iterations == 40
+    np.testing.assert_allclose(r.x.cpu().numpy(), ref.x.cpu().numpy(), rtol=1e-9, atol=1e-12)
+    y = torch.cat((r.y[:ns], r.y[more:more + nt]))
+    np.testing.assert_allclose(y.cpu().numpy(), ref.y.cpu().numpy(), rtol=1e-9, atol=1e-12)
+    assert not torch.any(r.y[ns:more]) and not torch.any(r.y[more + nt:])
+    del r, y
+    torch.cuda.empty_cache()
+
+
 def test_pdhg_internal_numbering_validates_endpoints(cuda, monkeypatch):
     """The library's own check (the Python wrapper validates first), on the numbering path."""
     from hello_ot_amd.lp.native_pdlp import run_pdhg
