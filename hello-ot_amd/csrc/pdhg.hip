@@ -795,14 +795,30 @@ __global__ __launch_bounds__(PT) void k_iteration(const Pdhg P, SidePlan src, Si
 // iteration s, each node it reads has used this workgroup's duals of iteration s - 1: the workgroup then sets them to
 // UNPUBLISHED again, waits until that store has reached memory, and publishes. A reader that has seen the new dual can
 // therefore only find UNPUBLISHED or a newer dual in the slot it reads next. All loads and stores of duals inside a
-// run have agent scope (they bypass the caches of the XCDs). All workgroups are on the chip at once (the launch is
-// cooperative), and a wait that lasts RESIDENT_WAIT ends the run with an error.
+// run have agent scope (they bypass the caches of the XCDs). All workgroups have to be on the chip at once: the launch is
+// cooperative, and where it is refused the solve goes on with separate launches. Where workgroups wait for one that is not
+// there all the same (CUs masked off the process, another process's run), a wait of ResidentSetting::wait ends the run,
+// and the solve starts again with separate launches.
 //
 // Measured, us per iteration, separate launches -> resident: 700 nodes a side and 6 thousand edges 5.2 -> 2.2, 4096 and
 // 61 thousand 8.7 -> 3.3, 16384 and 246 thousand 11.8 -> 7.8, where the gathers that bypass the caches (some 50 per ns)
 // bound it; a grid barrier instead of the signals took 6 at 4096 nodes, with a release fence that writes back L2 14.
 constexpr long long UNPUBLISHED = 0x7FF85E1DE0000001ll;  // a NaN that no operation returns
-constexpr long long RESIDENT_WAIT = 2000000000ll;         // 20 s of the 100 MHz clock
+
+// HELLOOT_PDHG_RESIDENT: "off" for separate launches alone, or the ticks of the 100 MHz clock a wait may last (default 2 s)
+struct ResidentSetting {
+    bool on;
+    long long wait;
+};
+inline ResidentSetting resident_setting() {
+    constexpr long long WAIT = 200000000ll;
+    const char* v = std::getenv("HELLOOT_PDHG_RESIDENT");
+    if (v == nullptr || *v == 0) return {true, WAIT};
+    if (std::strcmp(v, "off") == 0) return {false, WAIT};
+    char* end = nullptr;
+    const long long t = std::strtoll(v, &end, 10);
+    return {true, (end && *end == 0 && t >= 0) ? t : WAIT};
+}
 
 // part[0..ws]: first source node of each of the ws source workgroups (and n), then part[ws+1..]: the same for the
 // targets. Cut at equal weights of a side's nodes in order, a node weighing its degree + k.
@@ -841,12 +857,17 @@ __device__ __forceinline__ bool unpublished(double v) { return __double_as_longl
 template <int K>
 __global__ __launch_bounds__(RESIDENT_T, K > 4 ? 4 : 1) void k_resident(const Pdhg P, int ws, int steps, int64_t inner,
                                                                       double* cur, double* next, double* spare,
-                                                                      double primal_step, double dual_step) {
+                                                                      double primal_step, double dual_step,
+                                                                      long long wait) {
     constexpr int T = RESIDENT_T;
     __shared__ double refl[T * K];
     __shared__ double dual[T];
     __shared__ int late;
     const int tid = threadIdx.x;
+    // a workgroup that starts after the others gave up has nobody to wait for
+    if (tid == 0) late = __hip_atomic_load(P.result + 4, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0.0;
+    __syncthreads();
+    if (late) return;
     const bool source = (int)blockIdx.x < ws;
     const int b = source ? blockIdx.x : blockIdx.x + 1;
     const int32_t p0 = P.part[b], p1 = P.part[b + 1];
@@ -885,7 +906,6 @@ __global__ __launch_bounds__(RESIDENT_T, K > 4 ? 4 : 1) void k_resident(const Pd
         k0 = P.off[i] - ebase - e0;
         k1 = P.off[i + 1] - ebase - e0;
     }
-    if (tid == 0) late = 0;
     __syncthreads();
     for (int s = 0; s < steps; ++s) {
         double g[K];
@@ -910,7 +930,7 @@ __global__ __launch_bounds__(RESIDENT_T, K > 4 ? 4 : 1) void k_resident(const Pd
                             g[u] = __hip_atomic_load(cur + gi[u], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 #pragma unroll
                     for (int u = 0; u < K; ++u) miss |= unpublished(g[u]);
-                    if (wall_clock64() - from > RESIDENT_WAIT) {
+                    if (wall_clock64() - from > wait) {
                         late = 1;
                         break;
                     }
@@ -927,7 +947,7 @@ __global__ __launch_bounds__(RESIDENT_T, K > 4 ? 4 : 1) void k_resident(const Pd
         }
         __syncthreads();
         if (late) {
-            if (tid == 0) P.result[4] = 1.0;
+            if (tid == 0) __hip_atomic_store(P.result + 4, 1.0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             return;
         }
         if (tid < nn) {
@@ -996,14 +1016,20 @@ inline ResidentPlan resident_plan(int64_t n, int64_t nt, int64_t e, int max_s, i
 constexpr int64_t RESIDENT_STEPS = 16;
 constexpr int64_t RESIDENT_MOST = 4096;  // keeps a launch under some 50 ms
 
+// REFUSED: the runtime did not take the cooperative launch; `cur` and the state are as they were.
+constexpr int REFUSED = -1;
 int launch_resident(hipStream_t st, const Pdhg& P, const ResidentPlan& rp, int steps, int64_t inner, double* cur,
-                    double* next, double* spare, double ps, double ds) {
+                    double* next, double* spare, double ps, double ds, long long wait) {
     hipLaunchKernelGGL(k_unpublish, dim3(64), dim3(256), 0, st, next, spare, P.nodes);
     HM_LAUNCH_CHECK("k_unpublish");
     Pdhg p = P;
     int ws = rp.ws;
-    void* args[] = {&p, &ws, &steps, &inner, &cur, &next, &spare, &ps, &ds};
-    HM_HIP(hipLaunchCooperativeKernel(resident_kernel(rp.k), dim3(rp.ws + rp.wt), dim3(RESIDENT_T), args, 0, st));
+    void* args[] = {&p, &ws, &steps, &inner, &cur, &next, &spare, &ps, &ds, &wait};
+    if (hipLaunchCooperativeKernel(resident_kernel(rp.k), dim3(rp.ws + rp.wt), dim3(RESIDENT_T), args, 0, st) != hipSuccess) {
+        (void)hipGetLastError();
+        return REFUSED;
+    }
+    prof_count(rp.k == 2 ? "pdhg_resident_2" : rp.k == 4 ? "pdhg_resident_4" : "pdhg_resident_8", 1);
     return HM_OK;
 }
 
@@ -1122,56 +1148,22 @@ int number_nodes(hipStream_t st, const int64_t* rows, const int64_t* cols, int64
     return HM_OK;
 }
 
+constexpr int LATE = -2;  // a resident run gave up: its state is lost
 int read_result(hipStream_t st, const Pdhg& P, int q, double* host) {
     hipLaunchKernelGGL(k_combine, dim3(1), dim3(RT), 0, st, P.partial, P.result, q);
     HM_LAUNCH_CHECK("k_combine");
     HM_HIP(hipMemcpyAsync(host, P.result, sizeof(double) * 5, hipMemcpyDeviceToHost, st));
     HM_HIP(hipStreamSynchronize(st));
-    if (host[4] != 0.0) return fail(HM_EHIP, "PDHG: a workgroup of a resident run did not answer in time");
-    return HM_OK;
+    return host[4] != 0.0 ? LATE : HM_OK;
 }
 
-}  // namespace
-}  // namespace hm
-
-using namespace hm;
-
-extern "C" size_t hm_pdhg_workspace_bytes(int64_t n_source, int64_t n_target, int64_t e) {
-    if (n_source < 1 || n_target < 1 || e < 1) return 0;
-    Sizer s;
-    Pdhg P;
-    pdhg_layout(s, n_source, n_target, e, sort_tmp_bytes(n_source + n_target, e),
-                order_sort_tmp_bytes(n_source, n_target), P);
-    return s.used;
-}
-
-extern "C" int hm_pdhg_solve(void* stream, const int64_t* rows, const int64_t* cols, const double* costs,
-                             const double* masses, const double* x0, const double* y0, int64_t n_source,
-                             int64_t n_target, int64_t e, const hm_pdhg_params* params, double* x_out, double* y_out,
-                             hm_pdhg_result* result, void* workspace, size_t workspace_bytes) {
-    const auto started = std::chrono::steady_clock::now();
-    HM_CHECK_ARG(params && result, "PDHG: params and result are required");
-    HM_CHECK_ARG(n_source >= 1 && n_target >= 1 && e >= 1, "invalid restricted OT dimensions");
-    HM_CHECK_ARG(2 * e < INT32_MAX && n_source + n_target < INT32_MAX, "restricted OT too large for int32 indexing");
-    HM_CHECK_ARG(rows && cols && costs && masses && x_out && y_out, "PDHG: null pointer argument");
+// One solve on validated arguments, from the assembly on; LATE: start again without resident runs (the outputs are
+// written at the end alone).
+int pdhg_solve(hipStream_t st, const int64_t* rows, const int64_t* cols, const double* costs, const double* masses,
+               const double* x0, const double* y0, const hm_pdhg_params* params, double* x_out, double* y_out,
+               hm_pdhg_result* result, Pdhg& P, std::chrono::steady_clock::time_point started, ResidentSetting setting) {
+    const int64_t n = P.n, nt = P.nt, nodes = P.nodes, e = P.e;
     const int freq = params->evaluation_frequency;
-    HM_CHECK_ARG(freq >= 1 && params->iteration_limit >= 1 && params->time_limit_seconds > 0,
-                 "invalid restricted OT dimensions or runtime limits");
-    hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-    const int64_t n = n_source, nt = n_target, nodes = n + nt;
-    const size_t tmp = sort_tmp_bytes(nodes, e), otmp = order_sort_tmp_bytes(n, nt);
-    Sizer sz;
-    Pdhg P;
-    pdhg_layout(sz, n, nt, e, tmp, otmp, P);
-    HM_CHECK_ARG(workspace != nullptr, "workspace is required");
-    if (workspace_bytes < sz.used) return fail(HM_ENOSPC, "PDHG workspace too small: %zu < %zu", workspace_bytes, sz.used);
-    Arena a(workspace, workspace_bytes);
-    pdhg_layout(a, n, nt, e, tmp, otmp, P);
-    P.n = n;
-    P.nt = nt;
-    P.nodes = nodes;
-    P.e = e;
-
     // ---- LP assembly: node numbers, endpoints, degrees, per-node incident edge lists (ascending edge id) ----
     hipLaunchKernelGGL(k_fill_i32, dim3(grid_of(nodes + 1)), dim3(256), 0, st, P.deg, nodes + 1, 0);
     hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, st, P.flag, 4, 0);
@@ -1260,7 +1252,8 @@ extern "C" int hm_pdhg_solve(void* stream, const int64_t* rows, const int64_t* c
                            nt, tgt.npb, (int32_t)e, P.row_t, P.gbase_t, P.g16_t);
     }
     HM_LAUNCH_CHECK("node-block setup");
-    const ResidentPlan resident = resident_plan(n, nt, e, flag[1], flag[2]);
+    ResidentPlan resident{0, 0, 0};
+    if (setting.on) resident = resident_plan(n, nt, e, flag[1], flag[2]);
     if (resident.k > 0) {
         hipLaunchKernelGGL(k_partition, dim3(1), dim3(256), 0, st, P.off, n, nt, e, resident.ws, resident.wt, resident.k,
                            P.part);
@@ -1335,10 +1328,14 @@ extern "C" int hm_pdhg_solve(void* stream, const int64_t* rows, const int64_t* c
         const int64_t plain = freq - 1 - local_count % freq;  // iterations before the next major one
         const int64_t steps = plain < RESIDENT_MOST ? plain : RESIDENT_MOST;
         if (resident.k > 0 && !checkpoint && steps >= RESIDENT_STEPS) {
-            if (int rc = launch_resident(st, P, resident, (int)steps, local_inner, P.dual[at], P.dual[(at + 1) % 3],
-                                         P.dual[(at + 2) % 3], primal_step, dual_step))
-                return rc;
+            const int rc = launch_resident(st, P, resident, (int)steps, local_inner, P.dual[at], P.dual[(at + 1) % 3],
+                                           P.dual[(at + 2) % 3], primal_step, dual_step, setting.wait);
             prof_end(st);
+            if (rc == REFUSED) {  // separate launches from here on
+                resident.k = 0;
+                continue;
+            }
+            if (rc) return rc;
             prof_count("pdhg_iteration", steps - 1);
             at = (int)((at + steps) % 3);
             local_count += steps;
@@ -1379,4 +1376,55 @@ extern "C" int hm_pdhg_solve(void* stream, const int64_t* rows, const int64_t* c
     result->primal_weight = weight;
     result->seconds = std::chrono::duration<double>(std::chrono::steady_clock::now() - started).count();
     return HM_OK;
+}
+
+}  // namespace
+}  // namespace hm
+
+using namespace hm;
+
+extern "C" size_t hm_pdhg_workspace_bytes(int64_t n_source, int64_t n_target, int64_t e) {
+    if (n_source < 1 || n_target < 1 || e < 1) return 0;
+    Sizer s;
+    Pdhg P;
+    pdhg_layout(s, n_source, n_target, e, sort_tmp_bytes(n_source + n_target, e),
+                order_sort_tmp_bytes(n_source, n_target), P);
+    return s.used;
+}
+
+extern "C" int hm_pdhg_solve(void* stream, const int64_t* rows, const int64_t* cols, const double* costs,
+                             const double* masses, const double* x0, const double* y0, int64_t n_source,
+                             int64_t n_target, int64_t e, const hm_pdhg_params* params, double* x_out, double* y_out,
+                             hm_pdhg_result* result, void* workspace, size_t workspace_bytes) {
+    const auto started = std::chrono::steady_clock::now();
+    HM_CHECK_ARG(params && result, "PDHG: params and result are required");
+    HM_CHECK_ARG(n_source >= 1 && n_target >= 1 && e >= 1, "invalid restricted OT dimensions");
+    HM_CHECK_ARG(2 * e < INT32_MAX && n_source + n_target < INT32_MAX, "restricted OT too large for int32 indexing");
+    HM_CHECK_ARG(rows && cols && costs && masses && x_out && y_out, "PDHG: null pointer argument");
+    const int freq = params->evaluation_frequency;
+    HM_CHECK_ARG(freq >= 1 && params->iteration_limit >= 1 && params->time_limit_seconds > 0,
+                 "invalid restricted OT dimensions or runtime limits");
+    hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+    const int64_t n = n_source, nt = n_target, nodes = n + nt;
+    const size_t tmp = sort_tmp_bytes(nodes, e), otmp = order_sort_tmp_bytes(n, nt);
+    Sizer sz;
+    Pdhg P;
+    pdhg_layout(sz, n, nt, e, tmp, otmp, P);
+    HM_CHECK_ARG(workspace != nullptr, "workspace is required");
+    if (workspace_bytes < sz.used) return fail(HM_ENOSPC, "PDHG workspace too small: %zu < %zu", workspace_bytes, sz.used);
+    Arena a(workspace, workspace_bytes);
+    pdhg_layout(a, n, nt, e, tmp, otmp, P);
+    P.n = n;
+    P.nt = nt;
+    P.nodes = nodes;
+    P.e = e;
+    const ResidentSetting setting = resident_setting();
+    const Pdhg fresh = P;
+    int rc = pdhg_solve(st, rows, cols, costs, masses, x0, y0, params, x_out, y_out, result, P, started, setting);
+    if (rc == LATE) {
+        prof_count("pdhg_resident_late", 1);
+        P = fresh;
+        rc = pdhg_solve(st, rows, cols, costs, masses, x0, y0, params, x_out, y_out, result, P, started, {false, 0});
+    }
+    return rc;
 }

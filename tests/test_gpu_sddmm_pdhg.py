@@ -6,6 +6,7 @@ import pytest
 import torch
 
 import oracle
+from hello_ot_amd import _lib
 from hello_ot_amd.costs.pairs import lowrank_csr_costs, lowrank_pair_costs, norm_pair_costs
 from hello_ot_amd.lp import NativeRestrictedOTPDLP
 
@@ -406,21 +407,9 @@ def test_pdhg_with_internal_node_numbers_matches_oracle(cuda, monkeypatch, name)
     assert out["1"].obj_val == pytest.approx(out["off"].obj_val, rel=1e-12)
 
 
-@pytest.mark.parametrize("ns,nt,per_row,hub,freq,checks", [
-    (2, 3, 3, 0, 17, 3),          # the smallest: one workgroup a side, runs of exactly 16 iterations
-    (700, 300, 5, 0, 40, 3),      # 2 edges a thread, degrees of the two sides apart
-    (700, 700, 5, 490, 16, 3),    # runs of 15: separate launches
-    (700, 700, 5, 490, 40, 2),    # a hub that all but fills a workgroup of 2 edges a thread
-    (700, 700, 5, 600, 40, 2),    # one that needs 4
-    (3000, 2500, 4, 2030, 40, 2),  # one that all but fills a workgroup of 8
-    (3000, 2500, 4, 2045, 40, 2),  # one that no workgroup holds: separate launches
-    (4096, 4096, 12, 0, 40, 2),   # 4 edges a thread
-    (16384, 12000, 10, 30, 40, 2),  # 8 edges a thread, more than a workgroup per CU
-    (300, 300, 2, 0, 4200, 1),    # more iterations than one launch runs
-])
-def test_pdhg_resident_runs_match_oracle(cuda, ns, nt, per_row, hub, freq, checks):
-    """The iterations between checkpoints in one cooperative launch, over its shapes and the edges of their rules. The
-    last source and target have no edges where a side has more than 200 nodes; edge lists in random order; warm start."""
+def _resident_lp(ns, nt, per_row, hub, freq):
+    """A random support in random edge order, a target joined to `hub` sources, warm starts; the last source and target
+    have no edges where a side has more than 200 nodes."""
     rng = np.random.default_rng(ns + hub + freq)
     live_s, live_t = ns - (ns > 200), nt - (nt > 200)
     cols = [rng.choice(live_t, min(per_row, live_t), replace=False) for _ in range(live_s)]
@@ -439,6 +428,41 @@ def test_pdhg_resident_runs_match_oracle(cuda, ns, nt, per_row, hub, freq, check
     a /= a.sum()
     b /= b.sum()
     x0, y0 = rng.random(rows.size) / rows.size, 0.1 * rng.standard_normal(ns + nt)
+    return rows, cols, costs, a, b, x0, y0
+
+
+def _solve_resident(dev, lp, freq, checks):
+    """(result, resident launches with 2, 4 and 8 edges a thread, solves that started again without)"""
+    rows, cols, costs, a, b, x0, y0 = lp
+    _lib.profile_reset()
+    _lib.profile_enable(True)
+    try:
+        r = NativeRestrictedOTPDLP(device=dev, evaluation_frequency=freq, iteration_limit=freq * checks).solve_restricted(
+            rows=rows, cols=cols, costs=costs, source_mass=a, target_mass=b, tolerance=0.0, warm_start_primal=x0,
+            warm_start_dual=y0)
+        launches = [_lib.profile_query(f"pdhg_resident_{k}")[1] for k in (2, 4, 8)]
+        return r, launches, _lib.profile_query("pdhg_resident_late")[1]
+    finally:
+        _lib.profile_enable(False)
+
+
+@pytest.mark.parametrize("ns,nt,per_row,hub,freq,checks", [
+    (2, 3, 3, 0, 17, 3),          # the smallest: one workgroup a side, runs of exactly 16 iterations
+    (700, 300, 5, 0, 40, 3),      # 2 edges a thread, degrees of the two sides apart
+    (700, 700, 5, 490, 16, 3),    # runs of 15: separate launches
+    (700, 700, 5, 490, 40, 2),    # a hub that all but fills a workgroup of 2 edges a thread
+    (700, 700, 5, 600, 40, 2),    # one that needs 4
+    (3000, 2500, 4, 2030, 40, 2),  # one that all but fills a workgroup of 8
+    (3000, 2500, 4, 2045, 40, 2),  # one that no workgroup holds: separate launches
+    (4096, 4096, 12, 0, 40, 2),   # 4 edges a thread
+    (16384, 12000, 10, 30, 40, 2),  # 8 edges a thread, more than a workgroup per CU
+    (300, 300, 2, 0, 4200, 1),    # more iterations than one launch runs
+])
+def test_pdhg_resident_runs_match_oracle(cuda, ns, nt, per_row, hub, freq, checks):
+    """The iterations between checkpoints in one cooperative launch, over its shapes and the edges of their rules. The
+    last source and target have no edges where a side has more than 200 nodes; edge lists in random order; warm start."""
+    lp = _resident_lp(ns, nt, per_row, hub, freq)
+    rows, cols, costs, a, b, x0, y0 = lp
     ref = oracle.pdhg_solve(rows, cols, costs, a, b, warm_start_primal=x0, warm_start_dual=y0,
                             evaluation_frequency=freq, iteration_limit=freq * checks, tolerance=0.0)
     r = NativeRestrictedOTPDLP(device=cuda, evaluation_frequency=freq, iteration_limit=freq * checks).solve_restricted(
@@ -448,6 +472,25 @@ def test_pdhg_resident_runs_match_oracle(cuda, ns, nt, per_row, hub, freq, check
     assert r.solver_diag["restart_count"] == ref["restart_count"]
     np.testing.assert_allclose(r.x.cpu().numpy(), ref["x"], rtol=1e-9, atol=1e-12)
     np.testing.assert_allclose(r.y.cpu().numpy(), ref["y"], rtol=1e-9, atol=1e-12)
+
+
+def _assert_same_solve(got, want):
+    assert torch.equal(got.x, want.x) and torch.equal(got.y, want.y)
+    assert got.iterations == want.iterations and got.solver_diag["restart_count"] == want.solver_diag["restart_count"]
+    assert (got.obj_val, got.dual_obj_val, got.gap) == (want.obj_val, want.dual_obj_val, want.gap)
+
+
+def test_pdhg_resident_run_that_gives_up(cuda, monkeypatch):
+    """A resident run whose waits end (here at once, by a limit of 0 ticks) does not fail the solve: it starts again with
+    separate launches and gives their result, bit for bit."""
+    lp = _resident_lp(4096, 4096, 20, 0, 40)
+    monkeypatch.setenv("HELLOOT_PDHG_RESIDENT", "off")
+    want, launches, late = _solve_resident(cuda, lp, 40, 3)
+    assert launches == [0, 0, 0] and late == 0
+    monkeypatch.setenv("HELLOOT_PDHG_RESIDENT", "0")
+    got, launches, late = _solve_resident(cuda, lp, 40, 3)
+    assert launches == [0, 1, 0] and late == 1
+    _assert_same_solve(got, want)
 
 
 def test_pdhg_more_nodes_than_one_launch_of_both_sides_takes(cuda, monkeypatch):
