@@ -446,38 +446,78 @@ def _solve_resident(dev, lp, freq, checks):
         _lib.profile_enable(False)
 
 
-@pytest.mark.parametrize("ns,nt,per_row,hub,freq,checks", [
-    (2, 3, 3, 0, 17, 3),          # the smallest: one workgroup a side, runs of exactly 16 iterations
-    (700, 300, 5, 0, 40, 3),      # 2 edges a thread, degrees of the two sides apart
-    (700, 700, 5, 490, 16, 3),    # runs of 15: separate launches
-    (700, 700, 5, 490, 40, 2),    # a hub that all but fills a workgroup of 2 edges a thread
-    (700, 700, 5, 600, 40, 2),    # one that needs 4
-    (3000, 2500, 4, 2030, 40, 2),  # one that all but fills a workgroup of 8
-    (3000, 2500, 4, 2045, 40, 2),  # one that no workgroup holds: separate launches
-    (4096, 4096, 12, 0, 40, 2),   # 4 edges a thread
-    (16384, 12000, 10, 30, 40, 2),  # 8 edges a thread, more than a workgroup per CU
-    (300, 300, 2, 0, 4200, 1),    # more iterations than one launch runs
-])
-def test_pdhg_resident_runs_match_oracle(cuda, ns, nt, per_row, hub, freq, checks):
-    """The iterations between checkpoints in one cooperative launch, over its shapes and the edges of their rules. The
-    last source and target have no edges where a side has more than 200 nodes; edge lists in random order; warm start."""
-    lp = _resident_lp(ns, nt, per_row, hub, freq)
-    rows, cols, costs, a, b, x0, y0 = lp
-    ref = oracle.pdhg_solve(rows, cols, costs, a, b, warm_start_primal=x0, warm_start_dual=y0,
-                            evaluation_frequency=freq, iteration_limit=freq * checks, tolerance=0.0)
-    r = NativeRestrictedOTPDLP(device=cuda, evaluation_frequency=freq, iteration_limit=freq * checks).solve_restricted(
-        rows=rows, cols=cols, costs=costs, source_mass=a, target_mass=b, tolerance=0.0, warm_start_primal=x0,
-        warm_start_dual=y0)
-    assert r.iterations == ref["iterations"] == freq * checks
-    assert r.solver_diag["restart_count"] == ref["restart_count"]
-    np.testing.assert_allclose(r.x.cpu().numpy(), ref["x"], rtol=1e-9, atol=1e-12)
-    np.testing.assert_allclose(r.y.cpu().numpy(), ref["y"], rtol=1e-9, atol=1e-12)
-
-
 def _assert_same_solve(got, want):
     assert torch.equal(got.x, want.x) and torch.equal(got.y, want.y)
     assert got.iterations == want.iterations and got.solver_diag["restart_count"] == want.solver_diag["restart_count"]
     assert (got.obj_val, got.dual_obj_val, got.gap) == (want.obj_val, want.dual_obj_val, want.gap)
+
+
+@pytest.mark.parametrize("ns,nt,per_row,hub,freq,checks,edges", [
+    (2, 3, 3, 0, 17, 3, 2),           # the smallest: one workgroup a side, runs of exactly 16 iterations
+    (700, 300, 5, 0, 40, 3, 2),       # 2 edges a thread, degrees of the two sides apart
+    (700, 700, 5, 490, 16, 3, 0),     # runs of 15: separate launches
+    (600, 300, 3, 490, 40, 2, 2),     # a hub that all but fills a workgroup of 2 edges a thread
+    (700, 700, 5, 490, 40, 2, 4),     # one whose side no longer fits a workgroup per CU with 2
+    (700, 700, 5, 600, 40, 2, 4),     # one that needs 4
+    (1100, 100, 2, 990, 40, 2, 4),    # one that all but fills a workgroup of 4
+    (2100, 60, 1, 2020, 40, 2, 8),    # of 8
+    (3000, 2500, 4, 2030, 40, 2, 0),  # one whose side no longer fits the chip: separate launches
+    (3000, 2500, 4, 2045, 40, 2, 0),  # one that no workgroup holds: separate launches
+    (4096, 4096, 12, 0, 40, 2, 2),
+    (4096, 4096, 20, 0, 40, 2, 4),
+    (16384, 12000, 10, 30, 40, 2, 8),  # more than a workgroup per CU
+    (300, 300, 2, 0, 4200, 1, 2),     # more iterations than one launch runs
+])
+def test_pdhg_resident_runs_match_oracle(cuda, monkeypatch, ns, nt, per_row, hub, freq, checks, edges):
+    """The iterations between checkpoints in one cooperative launch (`edges` a thread on 256 CUs; 0: separate launches), over
+    its shapes and the edges of their rules: against the oracle, and bit for bit what separate launches give."""
+    lp = _resident_lp(ns, nt, per_row, hub, freq)
+    rows, cols, costs, a, b, x0, y0 = lp
+    ref = oracle.pdhg_solve(rows, cols, costs, a, b, warm_start_primal=x0, warm_start_dual=y0,
+                            evaluation_frequency=freq, iteration_limit=freq * checks, tolerance=0.0)
+    r, launches, late = _solve_resident(cuda, lp, freq, checks)
+    assert [n > 0 for n in launches] == [edges == k for k in (2, 4, 8)] and late == 0
+    assert r.iterations == ref["iterations"] == freq * checks
+    assert r.solver_diag["restart_count"] == ref["restart_count"]
+    np.testing.assert_allclose(r.x.cpu().numpy(), ref["x"], rtol=1e-9, atol=1e-12)
+    np.testing.assert_allclose(r.y.cpu().numpy(), ref["y"], rtol=1e-9, atol=1e-12)
+    monkeypatch.setenv("HELLOOT_PDHG_RESIDENT", "off")
+    separate, launches, _ = _solve_resident(cuda, lp, freq, checks)
+    assert launches == [0, 0, 0]
+    _assert_same_solve(r, separate)
+
+
+def test_pdhg_resident_runs_on_two_streams(cuda):
+    """Two LPs from two threads, each on a stream of its own, give what each gives alone."""
+    import threading
+
+    lps = [_resident_lp(4096, 4096, 20, 0, 40), _resident_lp(16384, 12000, 10, 30, 40)]
+
+    def solve(lp):
+        rows, cols, costs, a, b, x0, y0 = lp
+        return NativeRestrictedOTPDLP(device=cuda, evaluation_frequency=40, iteration_limit=400).solve_restricted(
+            rows=rows, cols=cols, costs=costs, source_mass=a, target_mass=b, tolerance=0.0, warm_start_primal=x0,
+            warm_start_dual=y0)
+
+    want = [solve(lp) for lp in lps]
+    torch.cuda.synchronize()
+    got = [[], []]
+
+    def work(t):
+        with torch.cuda.stream(torch.cuda.Stream(cuda)):
+            for _ in range(3):
+                got[t].append(solve(lps[t]))
+            torch.cuda.current_stream(cuda).synchronize()
+
+    threads = [threading.Thread(target=work, args=(t,)) for t in (0, 1)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for t in (0, 1):
+        assert len(got[t]) == 3
+        for r in got[t]:
+            _assert_same_solve(r, want[t])
 
 
 def test_pdhg_resident_run_that_gives_up(cuda, monkeypatch):
