@@ -62,8 +62,8 @@ __global__ __launch_bounds__(256) void sddmm_quad_kernel(const float* __restrict
     const int lane = threadIdx.x & 63, t = lane & 15, g = lane >> 4;
     const int64_t waves = (int64_t)gridDim.x * (blockDim.x >> 6);
     for (int64_t row = (int64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6); row < m; row += waves) {
-        const int32_t e1 = rowptr[row + 1];
-        int32_t e = rowptr[row] + g;
+        const uint32_t e1 = rowptr[row + 1];  // (unsigned: four past the last entry of 2^31 - 1 is still past it)
+        uint32_t e = (uint32_t)rowptr[row] + g;
         int32_t next = e < e1 ? col[e] : 0;
         for (; e < e1; e += 4) {
             const int64_t j = next;
@@ -110,7 +110,7 @@ __global__ __launch_bounds__(256) void sddmm_l2sq_csr_kernel(const float* __rest
             // U gathered Y rows in flight per step; each pair keeps the fixed lane order
             constexpr int U = 4;
             int32_t e = e0;
-            for (; e + U <= e1; e += U) {
+            for (; e1 - e >= U; e += U) {
                 const float* yp[U];
                 double a[U];
 #pragma unroll

@@ -34,6 +34,29 @@ def test_sddmm_csr_bit_exact(cuda, m, n, d, per_row):
     np.testing.assert_array_equal(out.cpu().numpy(), ref)
 
 
+@pytest.mark.parametrize("d", [4, 6])
+def test_sddmm_csr_of_the_most_entries_that_rowptr_counts(cuda, d):
+    """2^31 - 1 entries, the last rows of several lengths: the loops' steps past a row's end stay past it (rows of 16-byte
+    loads, and a wave per entry with x in registers)."""
+    nnz, m, n = 2 ** 31 - 1, 1 << 20, 1000
+    g = torch.Generator(device=cuda).manual_seed(1)
+    X, Y = torch.randn(m, d, generator=g, device=cuda), torch.randn(n, d, generator=g, device=cuda)
+    p, q = (X.double() ** 2).sum(1), (Y.double() ** 2).sum(1)
+    counts = np.array([1, 2, 3, 4, 5, 6, 7, 8, 9])
+    rowptr = np.concatenate([np.linspace(0, nnz - counts.sum(), m + 1 - counts.size).astype(np.int64),
+                             nnz - counts.sum() + np.cumsum(counts)]).astype(np.int32)
+    col = torch.randint(0, n, (nnz,), generator=g, device=cuda, dtype=torch.int32)
+    out = lowrank_csr_costs(X, Y, p, q, torch.as_tensor(rowptr, device=cuda), col, dot_scale=2.0)
+    for at in (0, int(rowptr[1]) - 500, int(rowptr[m // 2]) - 500, nnz - 1000):
+        entries = torch.arange(at, min(at + 1000, nnz), device=cuda)
+        rows = torch.searchsorted(torch.as_tensor(rowptr[1:], device=cuda), entries.int(), right=True)
+        cols = col[at:at + 1000].long()
+        # (the same fixed order of sums: bit for bit)
+        assert torch.equal(out[at:at + 1000], lowrank_pair_costs(X, Y, p, q, rows, cols, dot_scale=2.0))
+    del out, col
+    torch.cuda.empty_cache()
+
+
 def test_sddmm_csr_empty_rows_and_validation(cuda):
     rng = np.random.default_rng(1)
     X = rng.standard_normal((6, 8)).astype(np.float32)
