@@ -433,6 +433,9 @@ __device__ __forceinline__ float seed_threshold(const unsigned int* __restrict__
 // Measured, whole calls with k = 2, rows, columns and certificate, before (features in LDS, one row per thread held to 64
 // registers, per-pair certificate branches) and now: 262144 x 262144, l1, d = 8: 80.1 -> 38.9 ms (21.5 instructions per
 // pair at 39.3e12 lane operations a second are 37.6 ms); 30000 x 40961, l2, d = 50: 75-85 -> 5.9 ms (3.8 ms).
+// Violated scores beyond the slack are counted and summed for the whole step without branches, since a scan far from the
+// optimum has one in most votes. 131072 x 131072, l1, d = 8, a third of the pairs violated: 14.2 ms (10.2 with few); pair by
+// pair in the part for rare ones 36.4, and 23.2 with the certificate branching per pair.
 template <int KIND, int DR, int R, bool TAIL, bool FUSED, bool ST>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sweep_waves(DR, R)))) void norm_sweep(const float* __restrict__ X, SweepSide side, int64_t m,
                                                   int64_t n, int d, const double* __restrict__ rb,
@@ -502,7 +505,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sweep_waves
                                          5.9604644775390625e-08 * (1.0 + 1e-6) + 1e-37)
                                : 0.0f;
     double num64 = 0.0, den64[R];
-    unsigned int count = 0u;  // violated pairs of this lane's rows in one segment: fits 32 bits
+    unsigned int count = 0u;           // violated pairs of this lane's rows in one segment within the slack
+    unsigned long long wcount = 0ull;  // and those of the wave beyond the slack
     float cm[R];              // largest acc
 #pragma unroll
     for (int r = 0; r < R; ++r) {
@@ -600,9 +604,37 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sweep_waves
                     }
                 }
                 if (!hits) continue;
-                // rare: some lane has a pair that may matter; each pair of the step in turn
+                // some lane has a pair that may matter. Violated scores beyond the slack, of which a state far from the optimum
+                // has many, are counted and squared here; only list and column entries and scores within the slack go on
+                unsigned int todo = (1u << (J * R)) - 1u;  // pair e = u R + r
+                if constexpr (ST) {
+                    unsigned long long rare[J][R], any = 0ull;
+                    float tnum = 0.0f;
+#pragma unroll
+                    for (int r = 0; r < R; ++r) {
+                        const float slack = sSlack[r * T], thr = sThr[r * T];
+#pragma unroll
+                        for (int u = 0; u < J; ++u) {
+                            const float s32 = (col[u].g - cost_of<KIND>(acc[u][r])) + fi32[r];
+                            const bool over = s32 > slack;
+                            const float sp = over ? s32 : 0.0f;
+                            tnum = fmaf(sp, sp, tnum);
+                            wcount += (unsigned long long)__popcll(__ballot(over));
+                            rare[u][r] = __ballot(s32 > thr) | __ballot(fabsf(s32) <= slack);
+                            if (FUSED) rare[u][r] |= __ballot(s32 > col[u].thr);
+                            any |= rare[u][r];
+                        }
+                    }
+                    num64 += (double)tnum;
+                    if (!any) continue;
+                    todo = 0u;
+#pragma unroll
+                    for (int e = 0; e < J * R; ++e) todo |= rare[e / R][e % R] ? 1u << e : 0u;
+                }
+                // rare: each of those pairs in turn
 #pragma unroll 1
-                for (int e = 0; e < J * R; ++e) {
+                for (; todo != 0u; todo &= todo - 1u) {
+                    const int e = __builtin_ctz(todo);
                     float a = acc[0][0], f32 = fi32[0];
 #pragma unroll
                     for (int u = 0; u < J; ++u)
@@ -627,7 +659,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sweep_waves
                     }
                     const bool enters = s32 > sThr[r * T];
                     const float slack = sSlack[r * T];
-                    const bool near = ST && s32 > -slack;
+                    const bool near = ST && s32 > -slack && !(s32 > slack);
                     if (enters || near) {
                         const double cd = (double)c, fi = sF[r * T], gj = cb[j];
                         const double sig = TRANSPOSED ? (fi - cd) + gj : (gj - cd) + fi;
@@ -660,12 +692,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sweep_waves
                             for (int q = 0; q < R; ++q)
                                 if (q == r) low[q] = lo;
                         }
-                        // beyond the slack the fp32 score decides; within it the exact fp64 score does (the maximum
+                        // beyond the slack the fp32 score decided; within it the exact fp64 score does (the maximum
                         // comes from the exact row lists afterwards)
-                        if (ST && s32 > slack) {
-                            num64 = fma((double)s32, (double)s32, num64);
-                            ++count;
-                        } else if (near && sig > 0.0) {
+                        if (near && sig > 0.0) {
                             num64 = fma(sig, sig, num64);
                             ++count;
                         }
@@ -717,7 +746,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sweep_waves
     }
     if (ST) {
         const int lane = tid & 63, wave = tid >> 6;
-        double v[5] = {num64, den, (double)count, 0.0, (double)cmax};  // slot 3: exact row maximum later
+        // (slot 3: exact row maximum later)
+        double v[5] = {num64, den, (double)count + (lane == 0 ? (double)wcount : 0.0), 0.0, (double)cmax};
 #pragma unroll
         for (int e = 0; e < 5; ++e)
             for (int o = 32; o >= 1; o >>= 1) {

@@ -651,17 +651,21 @@ def test_norm_lists_of_tiny_costs(cuda, kind, scale):
         assert int(st[2]) == ost[2] and float(st[3]) == ost[3]
 
 
+@pytest.mark.parametrize("dense", [False, True])
 @pytest.mark.parametrize("kind,d", [(0, 3), (1, 8), (2, 20), (0, 32)])
-def test_norm_two_rows_per_thread_agree_with_one(cuda, kind, d):
+def test_norm_two_rows_per_thread_agree_with_one(cuda, kind, d, dense):
     """Large sides with short lists run two rows per thread and, with both directions, column lists on the row sweep;
     lists of 8 run one row per thread and two sweeps. The first two entries of the long lists are the short ones, and the
-    certificates differ by the order of their sums (1e-9: fp64 sums of per-tile fp32 sums of the same terms)."""
+    certificates differ by the order of their sums (1e-9: fp64 sums of per-tile fp32 sums of the same terms). `dense`:
+    about half of the pairs are violated."""
     g0 = torch.Generator(device=cuda).manual_seed(90 + d)
     m, n = 70001, 8300
     X = torch.rand(m, d, generator=g0, device=cuda)
     Y = torch.rand(n, d, generator=g0, device=cuda)
     f = 0.2 * d ** 0.5 * torch.rand(m, generator=g0, device=cuda, dtype=torch.float64)
     g = 0.2 * torch.rand(n, generator=g0, device=cuda, dtype=torch.float64)
+    if dense:
+        f += torch.cdist(X[:512].double(), Y[:512].double(), p=(1.0, float("inf"), 2.0)[kind]).median()
     short, long = pricing_norm(X, Y, f, g, 2, kind), pricing_norm(X, Y, f, g, 8, kind)
     for a, b in zip(short[:4], long[:4]):
         assert torch.equal(a, b[:, :2])
