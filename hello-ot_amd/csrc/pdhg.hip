@@ -57,6 +57,7 @@ constexpr int RESIDENT_BLOCKS = 1024;  // its most workgroups
 
 struct Pdhg {
     int64_t n, nt, nodes, e;
+    double variable;  // the variables' scale, sqrt(2)
     // edges, source order
     int32_t *row, *col, *perm;
     double *cs, *x, *ax, *px, *dx;
@@ -68,7 +69,8 @@ struct Pdhg {
     uint8_t *loc_s, *loc_t;
     // node-block passes: the other side's node each edge gathers from (col / row_t) as a 16-bit offset from its
     // block's smallest one, when the block's edges span fewer than 65536 nodes of that side (gbase = that
-    // smallest node), else gbase = -1 and the pass reads the 4-byte number
+    // smallest node); else, up to 2^24 nodes, as one word with the own node's byte (gbase = PACKED; the words take the
+    // place of keys_in, which the incidence sort has read); else gbase = -1 and the pass reads the 4-byte number and the byte
     uint16_t *g16_s, *g16_t;
     int32_t *gbase_s, *gbase_t;
     // nodes
@@ -192,11 +194,14 @@ constexpr int ORDER_ROUNDS = 6;  // neighbour-averaging rounds (each: sources fr
 // setup kernels
 // ---------------------------------------------------------------------------------------------------------
 // Per node block (one workgroup each): the range of the other side's nodes its edges gather from, and when it spans
-// fewer than 65536 nodes, each edge's gathered node as an offset from the smallest (Pdhg::g16_*, gbase_*). The
+// fewer than 65536 nodes, each edge's gathered node as an offset from the smallest, else with `others` up to 2^24 nodes
+// there the gathered node above the edge's own node in the block (Pdhg::g16_*, gbase_*). The
 // block's edges are [off[b * npb] - ebase, off[min((b + 1) * npb, nodes)] - ebase).
+constexpr int32_t PACKED = -2;
 __global__ __launch_bounds__(256) void k_gather_base(const int32_t* __restrict__ off, int64_t nodes, int npb,
-                                                     int32_t ebase, const int32_t* __restrict__ gidx,
-                                                     int32_t* __restrict__ gbase, uint16_t* __restrict__ g16) {
+                                                     int32_t ebase, int64_t others, const int32_t* __restrict__ gidx,
+                                                     const uint8_t* __restrict__ loc, int32_t* __restrict__ gbase,
+                                                     uint16_t* __restrict__ g16, uint32_t* __restrict__ pack) {
     __shared__ int32_t smin[256], smax[256];
     const int64_t b = blockIdx.x;
     const int64_t n0 = b * npb, n1 = n0 + npb < nodes ? n0 + npb : nodes;
@@ -220,9 +225,13 @@ __global__ __launch_bounds__(256) void k_gather_base(const int32_t* __restrict__
     lo = smin[0];
     hi = smax[0];
     const bool narrow = e1 > e0 && (int64_t)hi - (int64_t)lo < 65536;
-    if (threadIdx.x == 0) gbase[b] = narrow ? lo : -1;
-    if (narrow)
+    const bool packed = others <= (int64_t)1 << 24;
+    if (threadIdx.x == 0) gbase[b] = narrow ? lo : packed ? PACKED : -1;
+    if (narrow) {
         for (int32_t p = e0 + (int32_t)threadIdx.x; p < e1; p += 256) g16[p] = (uint16_t)(gidx[p] - lo);
+    } else if (packed) {
+        for (int32_t p = e0 + (int32_t)threadIdx.x; p < e1; p += 256) pack[p] = (uint32_t)gidx[p] << 8 | loc[p];
+    }
 }
 
 // low bits of each edge's node number (its index within a node block of mask + 1 nodes)
@@ -618,6 +627,7 @@ struct Side {
     double *x, *px, *dx;    // dx: the source side alone (the checkpoint deltas of the edges)
     const uint8_t* loc;
     const uint16_t* g16;
+    const uint32_t* pack;
     const int32_t* gbase;
 };
 
@@ -635,11 +645,17 @@ __device__ __forceinline__ double edge_step(const Side& sd, int32_t p, double ow
     return r;
 }
 
+// ns of a node of `degree` edges, as k_node_setup forms it (a square root less to wait for than a load, and 8 bytes a node
+// less for the last-level cache)
+__device__ __forceinline__ double node_scale(int32_t degree, double variable) {
+    return variable * sqrt((double)(degree > 1 ? degree : 1));
+}
+
 // a node's update from the sum of its reflections
 template <bool CHECKPOINT, bool STORE>
-__device__ __forceinline__ void node_step(const Pdhg& P, int64_t i, double sum, double dual_step, double halpern,
-                                          double keep, double* __restrict__ next) {
-    const double yi = P.y[i], nsi = P.ns[i];
+__device__ __forceinline__ void node_step(const Pdhg& P, int64_t i, int32_t degree, double sum, double dual_step,
+                                          double halpern, double keep, double* __restrict__ next) {
+    const double yi = P.y[i], nsi = node_scale(degree, P.variable);
     const double pyi = yi - dual_step * (sum / nsi - P.bs[i]);
     const double refl = 2.0 * pyi - yi;
     if (STORE) P.py[i] = pyi;
@@ -682,7 +698,7 @@ __device__ __forceinline__ void group_pass(const Pdhg& P, const Side& sd, int64_
             if (left > 0) sum = group_ordered_sum<G>(sum, r[u], left < G ? left : G);
         }
     }
-    if (g == 0) node_step<CHECKPOINT, STORE>(P, i, sum, dual_step, halpern, keep, next);
+    if (g == 0) node_step<CHECKPOINT, STORE>(P, i, k1 - k0, sum, dual_step, halpern, keep, next);
 }
 
 // sum + v[a] + v[a+1] + ... + v[b-1], added one by one in that order; the LDS reads go out eight at a time so that
@@ -731,17 +747,24 @@ __device__ __forceinline__ void block_pass(const Pdhg& P, const Side& sd, int64_
     double sum = 0.0;
     for (int32_t base = e0; base < e1; base += EB) {
         const int len = e1 - base < EB ? e1 - base : EB;
-        for (int q = tid; q < len; q += PT) {
-            const int32_t p = base + q;
-            const int32_t c = gb >= 0 ? gb + (int32_t)sd.g16[p] : sd.gidx[p];
-            lds.refl[q] = edge_step<SOURCE, CHECKPOINT, STORE>(sd, p, lds.dual[sd.loc[p]], other[c], primal_step, halpern,
-                                                               keep);
+        auto step = [&](int q, int l, int32_t c) {
+            lds.refl[q] = edge_step<SOURCE, CHECKPOINT, STORE>(sd, base + q, lds.dual[l], other[c], primal_step, halpern, keep);
+        };
+        if (gb >= 0) {
+            for (int q = tid; q < len; q += PT) step(q, sd.loc[base + q], gb + (int32_t)sd.g16[base + q]);
+        } else if (gb == PACKED) {
+            for (int q = tid; q < len; q += PT) {
+                const uint32_t w = sd.pack[base + q];
+                step(q, w & 255u, (int32_t)(w >> 8));
+            }
+        } else {
+            for (int q = tid; q < len; q += PT) step(q, sd.loc[base + q], sd.gidx[base + q]);
         }
         __syncthreads();
         sum = fold_in_order(lds.refl, (k0 > base ? k0 : base) - base, (k1 < base + len ? k1 : base + len) - base, sum);
         __syncthreads();
     }
-    if (tid < nn) node_step<CHECKPOINT, STORE>(P, n0 + tid, sum, dual_step, halpern, keep, next);
+    if (tid < nn) node_step<CHECKPOINT, STORE>(P, n0 + tid, k1 - k0, sum, dual_step, halpern, keep, next);
 }
 
 // How one side runs: lane groups of U edges per lane (u > 0), or node blocks (u = 0); its workgroups.
@@ -752,19 +775,23 @@ struct SidePlan {
 
 constexpr int GL = 8;  // lanes per group
 
-// One PDHG iteration: workgroups [0, src.blocks) run the source side, the rest the target side (the first `first` of them
-// in earlier launches). Small problems are bound by the latency of a launch and of each pass's chain of dependent loads
+// One PDHG iteration: workgroups [0, src.blocks) run the source side, the rest the target side; workgroup i of the launch is
+// number first + step * i. Small problems are bound by the latency of a launch and of each pass's chain of dependent loads
 // (offsets, edges, gathered dual, fold), which the two sides now share: 4096 nodes a side and 61 thousand edges take 10.0 us
-// an iteration, as two dependent launches they took 11.3. Large ones stream the edge state (524288 a side, 12.5 million
-// edges: 318 us, before 324).
+// an iteration, as two dependent launches they took 11.3.
+// Large ones stream the edge state, all of it in each iteration, and whether that fits the last-level cache (256 MB) decides:
+// every other iteration runs its workgroups backward, so that it begins with what the last one left there, where a stream in
+// one direction has always just lost what it needs next. The second dual buffer had taken 262144 nodes a side of degree 16
+// (some 250 MB) over that edge, to 82 to 95 us by placement from 83; backward, without ns and with packed indexes 78 to 85.
+// 524288 a side, 12 million edges: 325 -> 301 us, as two launches 330.
 template <bool CHECKPOINT, bool STORE>
-__global__ __launch_bounds__(PT) void k_iteration(const Pdhg P, SidePlan src, SidePlan tgt, int64_t first,
+__global__ __launch_bounds__(PT) void k_iteration(const Pdhg P, SidePlan src, SidePlan tgt, int64_t first, int64_t step,
                                                   const double* __restrict__ cur, double* __restrict__ next, double ps,
                                                   double ds, double h) {
     __shared__ BlockLds lds;
-    const int64_t b = first + blockIdx.x;
+    const int64_t b = first + step * (int64_t)blockIdx.x;
     if (b < src.blocks) {
-        const Side sd{0, P.n, P.n, 0, P.col, P.cs, P.ax, P.x, P.px, P.dx, P.loc_s, P.g16_s, P.gbase_s};
+        const Side sd{0, P.n, P.n, 0, P.col, P.cs, P.ax, P.x, P.px, P.dx, P.loc_s, P.g16_s, P.keys_in, P.gbase_s};
         if (src.u == 0) block_pass<true, CHECKPOINT, STORE>(P, sd, b, src.npb, cur, next, ps, ds, h, lds);
         else if (src.u == 1) group_pass<GL, 1, true, CHECKPOINT, STORE>(P, sd, b, cur, next, ps, ds, h);
         else if (src.u == 2) group_pass<GL, 2, true, CHECKPOINT, STORE>(P, sd, b, cur, next, ps, ds, h);
@@ -772,7 +799,7 @@ __global__ __launch_bounds__(PT) void k_iteration(const Pdhg P, SidePlan src, Si
     } else {
         const int64_t bt = b - src.blocks;
         const Side sd{P.n, P.nt, 0, (int32_t)P.e, P.row_t, P.cs_t, P.ax_t, P.x_t, P.px_t, nullptr, P.loc_t, P.g16_t,
-                      P.gbase_t};
+                      P.keys_in + P.e, P.gbase_t};
         if (tgt.u == 0) block_pass<false, CHECKPOINT, STORE>(P, sd, bt, tgt.npb, cur, next, ps, ds, h, lds);
         else if (tgt.u == 1) group_pass<GL, 1, false, CHECKPOINT, STORE>(P, sd, bt, cur, next, ps, ds, h);
         else if (tgt.u == 2) group_pass<GL, 2, false, CHECKPOINT, STORE>(P, sd, bt, cur, next, ps, ds, h);
@@ -1095,18 +1122,20 @@ inline SidePlan side_plan(int64_t e, int64_t nodes, int max_degree) {
 // One PDHG iteration from the duals of `cur` to those of `next`. px / py are stored only on major iterations: they are
 // read only by the evaluation that follows one.
 int launch_iteration(hipStream_t st, const Pdhg& P, const SidePlan& src, const SidePlan& tgt, const double* cur,
-                     double* next, bool checkpoint, bool major, double ps, double ds, double h) {
+                     double* next, bool backward, bool checkpoint, bool major, double ps, double ds, double h) {
     // (a launch of 2^32 threads or more runs some of them; the lane groups take 8 a node)
     constexpr int64_t MOST = (int64_t)UINT32_MAX / PT;
     const int64_t blocks = src.blocks + tgt.blocks;
-    for (int64_t first = 0; first < blocks; first += MOST) {
-        const dim3 grid((unsigned)(blocks - first < MOST ? blocks - first : MOST)), block(PT);
+    const int64_t step = backward ? -1 : 1;
+    for (int64_t done = 0; done < blocks; done += MOST) {
+        const int64_t first = backward ? blocks - 1 - done : done;
+        const dim3 grid((unsigned)(blocks - done < MOST ? blocks - done : MOST)), block(PT);
         if (major)
-            hipLaunchKernelGGL((k_iteration<true, true>), grid, block, 0, st, P, src, tgt, first, cur, next, ps, ds, h);
+            hipLaunchKernelGGL((k_iteration<true, true>), grid, block, 0, st, P, src, tgt, first, step, cur, next, ps, ds, h);
         else if (checkpoint)
-            hipLaunchKernelGGL((k_iteration<true, false>), grid, block, 0, st, P, src, tgt, first, cur, next, ps, ds, h);
+            hipLaunchKernelGGL((k_iteration<true, false>), grid, block, 0, st, P, src, tgt, first, step, cur, next, ps, ds, h);
         else
-            hipLaunchKernelGGL((k_iteration<false, false>), grid, block, 0, st, P, src, tgt, first, cur, next, ps, ds, h);
+            hipLaunchKernelGGL((k_iteration<false, false>), grid, block, 0, st, P, src, tgt, first, step, cur, next, ps, ds, h);
     }
     HM_LAUNCH_CHECK("pdhg iteration");
     return HM_OK;
@@ -1206,7 +1235,7 @@ int pdhg_solve(hipStream_t st, const int64_t* rows, const int64_t* cols, const d
     const bool rescale = params->rescale != 0;
     const double bound = rescale ? 1.0 / std::max(1.0, mass_norm) : 1.0;
     const double objective = rescale ? 1.0 / std::max(1.0, cost_norm) : 1.0;
-    const double variable = std::sqrt(2.0);
+    const double variable = P.variable = std::sqrt(2.0);
     // source-order edge state and its target-order mirror
     hipLaunchKernelGGL(k_source_setup, dim3(grid_of(e)), dim3(256), 0, st, P.eid, e, rows, cols, costs, x0, bound,
                        objective, variable, P);
@@ -1244,12 +1273,12 @@ int pdhg_solve(hipStream_t st, const int64_t* rows, const int64_t* cols, const d
     if (src.u == 0) {
         hipLaunchKernelGGL(k_low_bits, dim3(grid_of(e)), dim3(256), 0, st, P.row, e, src.npb - 1, P.loc_s);
         hipLaunchKernelGGL(k_gather_base, dim3((unsigned)((n + src.npb - 1) / src.npb)), dim3(256), 0, st, P.off, n,
-                           src.npb, 0, P.col, P.gbase_s, P.g16_s);
+                           src.npb, 0, nt, P.col, P.loc_s, P.gbase_s, P.g16_s, P.keys_in);
     }
     if (tgt.u == 0) {
         hipLaunchKernelGGL(k_low_bits, dim3(grid_of(e)), dim3(256), 0, st, P.col_t, e, tgt.npb - 1, P.loc_t);
         hipLaunchKernelGGL(k_gather_base, dim3((unsigned)((nt + tgt.npb - 1) / tgt.npb)), dim3(256), 0, st, P.off + n,
-                           nt, tgt.npb, (int32_t)e, P.row_t, P.gbase_t, P.g16_t);
+                           nt, tgt.npb, (int32_t)e, n, P.row_t, P.loc_t, P.gbase_t, P.g16_t, P.keys_in + e);
     }
     HM_LAUNCH_CHECK("node-block setup");
     ResidentPlan resident{0, 0, 0};
@@ -1342,8 +1371,8 @@ int pdhg_solve(hipStream_t st, const int64_t* rows, const int64_t* cols, const d
             local_inner += steps;
             continue;
         }
-        if (int rc = launch_iteration(st, P, src, tgt, P.dual[at], P.dual[at == 0], checkpoint, major, primal_step, dual_step,
-                                      halpern))
+        if (int rc = launch_iteration(st, P, src, tgt, P.dual[at], P.dual[at == 0], (local_count & 1) != 0, checkpoint, major,
+                                      primal_step, dual_step, halpern))
             return rc;
         at = at == 0;
         prof_end(st);

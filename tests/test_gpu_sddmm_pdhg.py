@@ -333,6 +333,35 @@ def test_pdhg_node_blocks_with_16_bit_gather_offsets_match_oracle(cuda, monkeypa
     np.testing.assert_allclose(r.y.cpu().numpy(), ref["y"], rtol=1e-9, atol=1e-12)
 
 
+@pytest.mark.parametrize("side", ["source", "target"])
+def test_pdhg_node_blocks_with_each_form_of_gather_index(cuda, monkeypatch, side):
+    """Node blocks whose edges gather from nodes next to each other (16-bit offsets), up to 2^24 nodes (words of node and
+    byte) and beyond (4-byte numbers): the same LP with its far nodes spread out. Every per-node and per-edge operation is
+    the same; the norm sums, which set the weights, add in another order."""
+    monkeypatch.setenv("HELLOOT_PDHG_REORDER", "off")
+    rng = np.random.default_rng(8)
+    near, far, per = 300, 2600, 40
+    rows = np.concatenate([np.repeat(np.arange(near), per), rng.integers(0, near, far)])
+    cols = np.concatenate([rng.integers(0, far, near * per), np.arange(far)])
+    costs = rng.random(rows.size)
+    a, b = rng.random(near), rng.random(far)
+    a, b = a / a.sum(), b / b.sum()
+    out = []
+    for stride in (1, 100, 7000):
+        nodes = (far - 1) * stride + 1
+        assert (nodes >= 1 << 24) == (stride == 7000)
+        spread = torch.zeros(nodes, dtype=torch.float64, device=cuda)
+        spread[::stride] = torch.as_tensor(b, device=cuda)
+        ends, masses = [rows, cols * stride], [torch.as_tensor(a, device=cuda), spread]
+        if side == "target":
+            ends, masses = ends[::-1], masses[::-1]
+        r = NativeRestrictedOTPDLP(device=cuda, evaluation_frequency=20, iteration_limit=60).solve_restricted(
+            rows=ends[0], cols=ends[1], costs=costs, source_mass=masses[0], target_mass=masses[1], tolerance=0.0)
+        out.append(r)
+        np.testing.assert_allclose(r.x.cpu().numpy(), out[0].x.cpu().numpy(), rtol=1e-9, atol=1e-12)
+        assert r.solver_diag["restart_count"] == out[0].solver_diag["restart_count"]
+
+
 def test_pdhg_c3_shape_1000_iterations_against_oracle(cuda):
     """C3 structure (16 sorted uniform columns per row, uniform marginals, SDDMM costs), 1000 iterations,
     at m = n = 8192 where the CPU oracle finishes in seconds."""
