@@ -10,7 +10,7 @@
 // One thread owns one or two X rows (features in registers up to d = 128); a Y row is the same for the whole wave, so
 // its features are scalar loads and enter the vector instructions as scalar operands. Per pair the loop computes the
 // cost and one test against the lowest of the row's, the column's and the certificate's thresholds; what passes (a few
-// pairs in a thousand) is handled out of line, with the row lists in LDS. The certificate adds the squares of violated
+// pairs in a thousand) is handled out of line, with the row lists in LDS (long ones in memory, see norm_plan). The certificate adds the squares of violated
 // scores in fp64 and those of all costs in fp32, flushed to fp64 per tile or more often (cost_span).
 //
 // Column lists, k <= 2 with rows and columns requested: they ride on the row sweep, so every pair is evaluated
@@ -321,7 +321,7 @@ __device__ __forceinline__ void column_enter(const ColArgs& ca, SlotRun& run, bo
     if ((threadIdx.x & 63) == 0 && t > *thr) *thr = t;
 }
 
-// dynamic LDS of a sweep workgroup of T threads, R rows each, lists of k entries; fused sweeps add the columns' own
+// dynamic LDS of a sweep workgroup of T threads, R rows each, lists of k entries there; fused sweeps add the columns' own
 // values
 inline size_t sweep_lds(int T, int R, int k, bool fused) {
     return (size_t)R * T * (sizeof(double) + 3 * sizeof(float) + (size_t)k * (sizeof(double) + sizeof(int))) +
@@ -436,7 +436,7 @@ __device__ __forceinline__ float seed_threshold(const unsigned int* __restrict__
 // Violated scores beyond the slack are counted and summed for the whole step without branches, since a scan far from the
 // optimum has one in most votes. 131072 x 131072, l1, d = 8, a third of the pairs violated: 14.2 ms (10.2 with few); pair by
 // pair in the part for rare ones 36.4, and 23.2 with the certificate branching per pair.
-template <int KIND, int DR, int R, bool TAIL, bool FUSED, bool ST>
+template <int KIND, int DR, int R, bool TAIL, bool FUSED, bool ST, bool GL>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sweep_waves(DR, R)))) void norm_sweep(const float* __restrict__ X, SweepSide side, int64_t m,
                                                   int64_t n, int d, const double* __restrict__ rb,
                                                   const double* __restrict__ cb,
@@ -452,16 +452,22 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sweep_waves
     __shared__ double sRed[4][5];
     const int T = blockDim.x;
     const int tid = threadIdx.x;
+    const int kl = GL ? 0 : k;  // list entries in LDS
+    const int ls = GL ? 1 : T;  // between the entries of a list
     double* const sF = smem + tid;                                  // [R][T] row duals
-    double* const sV = smem + (size_t)R * T + tid;                  // [R][k][T] list scores
-    int* const sI = reinterpret_cast<int*>(smem + (size_t)R * T * (1 + k)) + tid;  // [R][k][T] list indices
-    float* const sThr = reinterpret_cast<float*>(sI - tid + (size_t)R * T * k) + tid;  // [R][T] list entry thresholds
+    double* sV = smem + (size_t)R * T + tid;                        // [R][k][T] list scores
+    int* sI = reinterpret_cast<int*>(smem + (size_t)R * T * (1 + kl)) + tid;  // [R][k][T] list indices
+    float* const sThr = reinterpret_cast<float*>(sI - tid + (size_t)R * T * kl) + tid;  // [R][T] list entry thresholds
     float* const sSlack = sThr + R * T;                             // [R][T] certificate slacks
     int* const sWorst = reinterpret_cast<int*>(sSlack + R * T);     // [R][T] place of the list's worst entry
     TileCol* const sG = reinterpret_cast<TileCol*>(sWorst - tid + R * T);  // [NT + 8]
     unsigned long long* const sOwn = reinterpret_cast<unsigned long long*>(sG + NT + 8);  // [2][NT], fused
     const int64_t row0 = (int64_t)blockIdx.x * (T * R) + tid;       // rows row0 + r T
     const int64_t seg = blockIdx.y;
+    if constexpr (GL) {  // [R][T][k], in place
+        sV = part_v + (seg * m + row0) * k;
+        sI = part_i + (seg * m + row0) * k;
+    }
     const int64_t y_begin = seg * seg_len;
     const int64_t y_end = y_begin + seg_len < n ? y_begin + seg_len : n;
     const double ymax1 = key_double(ymaxima[0]);
@@ -495,9 +501,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sweep_waves
         sThr[r * T] = thr;
         sSlack[r * T] = slack;
         sWorst[r * T] = 0;
-        for (int s = 0; s < k; ++s) {
-            sV[(r * k + s) * T] = -INFINITY;
-            sI[(r * k + s) * T] = -1;
+        for (int s = 0; s < k && (!GL || ok); ++s) {
+            sV[(size_t)r * k * T + s * ls] = -INFINITY;
+            sI[(size_t)r * k * T + s * ls] = -1;
         }
     }
     // the same bound over every pair of a column (row side at its maxima)
@@ -666,17 +672,17 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sweep_waves
                         double* const v = sV + (size_t)r * k * T;
                         int* const id = sI + (size_t)r * k * T;
                         const int w = sWorst[r * T];
-                        if (enters && sig == sig && better(sig, (int)j, v[w * T], id[w * T])) {
+                        if (enters && sig == sig && better(sig, (int)j, v[w * ls], id[w * ls])) {
                             // the list is unordered: the new entry replaces the worst, and the worst of the rest is found by
                             // independent reads (a sorted insertion is a chain of dependent ones)
-                            v[w * T] = sig;
-                            id[w * T] = (int)j;
+                            v[w * ls] = sig;
+                            id[w * ls] = (int)j;
                             double kth = v[0];
                             int kid = id[0], at = 0;
 #pragma unroll 4
                             for (int s = 1; s < k; ++s) {
-                                const double vs = v[s * T];
-                                const int is = id[s * T];
+                                const double vs = v[s * ls];
+                                const int is = id[s * ls];
                                 if (better(kth, kid, vs, is)) {
                                     kth = vs;
                                     kid = is;
@@ -722,7 +728,25 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sweep_waves
             int* oi = part_i + (seg * m + row) * k;
             double* const v = sV + (size_t)r * k * T;
             int* const id = sI + (size_t)r * k * T;
-            for (int s = 0; s < k; ++s) {  // in order, best first
+            for (int s = 0; GL && s + 1 < k; ++s) {  // in order, best first
+                double bv = v[s];
+                int bi = id[s], at = s;
+#pragma unroll 4
+                for (int q = s + 1; q < k; ++q) {
+                    const double vq = v[q];
+                    const int iq = id[q];
+                    if (better(vq, iq, bv, bi)) {
+                        bv = vq;
+                        bi = iq;
+                        at = q;
+                    }
+                }
+                v[at] = v[s];
+                id[at] = id[s];
+                v[s] = bv;
+                id[s] = bi;
+            }
+            for (int s = 0; !GL && s < k; ++s) {
                 double bv = v[0];
                 int bi = id[0], at = 0;
 #pragma unroll 4
@@ -999,9 +1023,11 @@ __global__ void norm_zero(unsigned long long* p, int count) {
     if ((int)threadIdx.x < count) p[threadIdx.x] = 0ull;
 }
 
+constexpr int GLOBAL_FEATURES = 32;  // longest rows whose sweeps also come with lists outside LDS
 // One sweep direction: S segments of seg_len columns; workgroups of T threads with R rows each.
 struct NormPlan {
     int S, R, T;
+    bool global;  // lists in their place in the partial lists
     int64_t seg_len;
 };
 
@@ -1018,23 +1044,32 @@ inline NormPlan norm_segments(int64_t rows, int64_t cols, int64_t rows_per_block
     p.S = (int)((cols + p.seg_len - 1) / p.seg_len);
     p.R = 1;
     p.T = NB_ROWS;
+    p.global = false;
     return p;
 }
 
 // The fp64 sweep: 256 threads, one row each. The fp32 sweep: two rows per thread share the loads and tests of a Y row
-// where their features fit the registers beside enough waves (d <= 32) and the problem still fills the chip; 128
-// threads for lists of more than 16 entries (their LDS). Its partial lists take no more than those of one row per
-// thread, or 24 MiB.
+// where their features fit the registers beside enough waves (d <= 32) and the problem still fills the chip. Its partial
+// lists take no more than those of one row per thread, or 24 MiB.
+// Lists in LDS, 12 k bytes a row, leave few waves on a CU (8 at k = 16, 6 at k = 32), too few for a pair loop of few
+// features; in their place in the partial lists, in memory, an entry costs more and a pair less. Top-16 (top-32) rows, l1, in
+// LDS and in memory, d = 8: 65536 x 65536 16.8 and 14.1 ms (55 and 43), 262144 x 262144 99 and 58 (273 and 120),
+// 524288 x 524288 379 and 200 (894 and 332); d = 32: 65536 x 65536 19.1 and 16.0. Lists of 5 to 8 are level at
+// 131072 x 131072 (13.3 and 13.7) and behind below (65536: 5.1 and 5.8); 180000 x 180000 32.1 and 20.8, 524288 x 524288 183
+// and, with two rows per thread, 128. Rows of more than 32 features keep LDS, with 128 threads for lists of more than 16.
 inline NormPlan norm_plan(int64_t rows, int64_t cols, int d, int k, uint32_t flags) {
     const NormPlan one = norm_segments(rows, cols, NB_ROWS, 64);
     if (flags & HM_FP64) return one;
-    const int T = k > 16 ? 128 : 256;
-    const int R = (d <= 32 && k <= 4 && ((rows + 511) / 512) * ((cols + NT - 1) / NT) >= 4096) ? 2 : 1;
+    const bool global = d <= GLOBAL_FEATURES && (k > 8 || (k > 4 && d <= 8 && rows > (int64_t(1) << 34) / cols));
+    const int T = k > 16 && !global ? 128 : 256;
+    const bool fills = ((rows + 511) / 512) * ((cols + NT - 1) / NT) >= 4096;
+    const int R = d <= 32 && ((k <= 4 && fills) || (global && k <= 8 && rows >= 524288)) ? 2 : 1;
     int64_t most = (int64_t(24) << 20) / (12 * rows * k);
     if (most < one.S) most = one.S;
     NormPlan p = norm_segments(rows, cols, (int64_t)T * R, most < 64 ? most : 64);
     p.R = R;
     p.T = T;
+    p.global = global;
     return p;
 }
 
@@ -1150,16 +1185,25 @@ template <int KIND, int DR, int R, bool TAIL>
 int norm_direction_t(hipStream_t st, const Direction& D, int d, int k, const NormWork& w, double* stats_out, int linf) {
     const int64_t rows = (int64_t)D.plan.T * R;
     const dim3 grid((unsigned)((D.m + rows - 1) / rows), (unsigned)D.plan.S), block((unsigned)D.plan.T);
-    const size_t shmem = sweep_lds(D.plan.T, R, k, D.cols.gthr != nullptr);
+    const size_t shmem = sweep_lds(D.plan.T, R, D.plan.global ? 0 : k, D.cols.gthr != nullptr);
     const SweepSide side{D.Y, D.tail, tail_start(D.n, d)};
     prof_begin(st, D.gate != nullptr ? "norm_sweep_swapped" : "norm_sweep");
-#define HM_NORM_SWEEP(FUSED, ST)                                                                                    \
-    hipLaunchKernelGGL((norm_sweep<KIND, DR, R, TAIL, FUSED, ST>), grid, block, shmem, st, D.X, side, D.m, D.n, d, D.rb, \
+#define HM_NORM_SWEEP(FUSED, ST, GL)                                                                                \
+    hipLaunchKernelGGL((norm_sweep<KIND, DR, R, TAIL, FUSED, ST, GL>), grid, block, shmem, st, D.X, side, D.m, D.n, d, D.rb, \
                        D.cb, D.ymaxima, k, D.plan.seg_len, w.pv, w.pi, w.bs, (int)D.transposed, D.seeds, D.cols, D.gate, D.gate_cap)
     // (a fused call without the certificate takes the same kernel and leaves its sums unread)
-    if (D.cols.gthr != nullptr) HM_NORM_SWEEP(true, true);
-    else if (D.stats) HM_NORM_SWEEP(false, true);
-    else HM_NORM_SWEEP(false, false);
+    bool done = false;
+    if constexpr (DR > 0 && DR <= GLOBAL_FEATURES) {
+        if (D.plan.global) {
+            if (D.stats) HM_NORM_SWEEP(false, true, true);
+            else HM_NORM_SWEEP(false, false, true);
+            done = true;
+        }
+    }
+    if (done) {
+    } else if (D.cols.gthr != nullptr) HM_NORM_SWEEP(true, true, false);
+    else if (D.stats) HM_NORM_SWEEP(false, true, false);
+    else HM_NORM_SWEEP(false, false, false);
 #undef HM_NORM_SWEEP
     prof_end(st);
     HM_LAUNCH_CHECK("norm_sweep");

@@ -675,6 +675,26 @@ def test_norm_two_rows_per_thread_agree_with_one(cuda, kind, d, dense):
 
 
 @pytest.mark.parametrize("kind", [0, 1, 2])
+@pytest.mark.parametrize("m,n,d", [(140001, 130001, 7), (524288 + 77, 33001, 3)])
+def test_norm_lists_in_memory_agree_with_lists_in_lds(cuda, kind, m, n, d):
+    """Above 2^34 pairs lists of 5 to 8 entries lie in memory (with two rows per thread from 524288 rows on), as lists of
+    more than 8 do at any size; lists of 4 lie in LDS. Each holds the shorter one's entries first; the certificates differ
+    by the order of their sums (1e-9)."""
+    g0 = torch.Generator(device=cuda).manual_seed(7 + d)
+    X = torch.rand(m, d, generator=g0, device=cuda)
+    Y = torch.rand(n, d, generator=g0, device=cuda)
+    f = 0.1 * torch.rand(m, generator=g0, device=cuda, dtype=torch.float64)
+    g = 0.1 * torch.rand(n, generator=g0, device=cuda, dtype=torch.float64)
+    lists = [pricing_norm(X, Y, f, g, k, kind, cols=False) for k in (4, 8, 9)]
+    for short, long in zip(lists, lists[1:]):
+        k = short[0].shape[1]
+        assert torch.equal(short[0], long[0][:, :k]) and torch.equal(short[1], long[1][:, :k])
+        a, b = short[4].cpu().numpy(), long[4].cpu().numpy()
+        assert a[2] == b[2] and a[3] == b[3] and a[4] == b[4]
+        np.testing.assert_allclose(a[:2], b[:2], rtol=1e-9)
+
+
+@pytest.mark.parametrize("kind", [0, 1, 2])
 @pytest.mark.parametrize("k,grid", [(2, False), (1, False), (2, True)])
 def test_norm_fused_columns_overflow_and_two_sweep_paths_agree(cuda, kind, k, grid):
     """k <= 2 bidirectional calls evaluate each pair once and collect the column lists through the candidate buffer.
