@@ -777,7 +777,7 @@ constexpr int GL = 8;  // lanes per group
 
 // One PDHG iteration: workgroups [0, src.blocks) run the source side, the rest the target side; workgroup i of the launch is
 // number first + step * i. Small problems are bound by the latency of a launch and of each pass's chain of dependent loads
-// (offsets, edges, gathered dual, fold), which the two sides now share: 4096 nodes a side and 61 thousand edges take 10.0 us
+// (offsets, edges, gathered dual, fold), which the two sides now share: 4096 nodes a side and 82 thousand edges take 10.0 us
 // an iteration, as two dependent launches they took 11.3.
 // Large ones stream the edge state, all of it in each iteration, and whether that fits the last-level cache (256 MB) decides:
 // every other iteration runs its workgroups backward, so that it begins with what the last one left there, where a stream in
@@ -810,8 +810,10 @@ __global__ __launch_bounds__(PT) void k_iteration(const Pdhg P, SidePlan src, Si
 // ---------------------------------------------------------------------------------------------------------
 // resident runs of iterations
 // ---------------------------------------------------------------------------------------------------------
-// Up to some 2 million edges and nodes the whole iteration state fits the chip's registers, and an iteration of separate
-// launches is bound by latency: the launch, then offsets, edges, gathered duals, each from memory. A resident run does
+// While the two mirrored copies of the edges, and 8 for each node, fit RESIDENT_BLOCKS workgroups of 2048 less the largest
+// degree (resident_plan: 2 e + 8 nodes <= 1024 * (2039 - degree), some 0.6 million edges at a mean degree of 15), the whole
+// iteration state fits the chip's registers, and an iteration of separate launches is bound by latency: the launch, then
+// offsets, edges, gathered duals, each from memory. A resident run does
 // the plain iterations between two checkpoints in one cooperative launch: each workgroup keeps the edges of a run of
 // consecutive nodes of one side in registers (iterate, anchor, cost, gathered node) and its nodes' duals in LDS, and
 // only the duals that other workgroups gather pass through memory.
@@ -827,9 +829,10 @@ __global__ __launch_bounds__(PT) void k_iteration(const Pdhg P, SidePlan src, Si
 // there all the same (CUs masked off the process, another process's run), a wait of ResidentSetting::wait ends the run,
 // and the solve starts again with separate launches.
 //
-// Measured, us per iteration, separate launches -> resident: 700 nodes a side and 6 thousand edges 5.2 -> 2.2, 4096 and
-// 61 thousand 8.7 -> 3.3, 16384 and 246 thousand 11.8 -> 7.8, where the gathers that bypass the caches (some 50 per ns)
-// bound it; a grid barrier instead of the signals took 6 at 4096 nodes, with a release fence that writes back L2 14.
+// Measured, 1000 iterations with set-up and checks, separate launches -> resident: 700 nodes a side and 6.6 thousand edges
+// 6.4 -> 3.3 ms, 4096 and 82 thousand 10.1 -> 4.6, 16384 and 328 thousand 12.9 -> 9.3, 24000 and 480 thousand 17.5 -> 13.5,
+// where the gathers that bypass the caches (some 50 per ns) bound it; at 4096 nodes an iteration with a grid barrier instead
+// of the signals took 6 us, with a release fence that writes back L2 14.
 constexpr long long UNPUBLISHED = 0x7FF85E1DE0000001ll;  // a NaN that no operation returns
 
 // HELLOOT_PDHG_RESIDENT: "off" for separate launches alone, or the ticks of the 100 MHz clock a wait may last (default 2 s)

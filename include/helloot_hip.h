@@ -142,7 +142,7 @@ int hm_pricing_l2sq_resident_floor(void* stream, const float* X, const float* Y,
  * direct_norm_fp64, cost.cu:84-104): per pair every feature difference in fp64 from the fp32 inputs, combined in
  * feature order (l1 sum|z|, linf max|z|, l2 sqrt of fma(z, z, acc)); scores and certificate are then fp64 throughout
  * and the column lists come from a second, role-swapped sweep.
- * With k <= 2 and both HM_ROWS and HM_COLS, the column lists come from the row sweep through a candidate buffer in
+ * With k <= 2, both HM_ROWS and HM_COLS and m <= 32 n, the column lists come from the row sweep through a candidate buffer in
  * the workspace: hm_pricing_norm_workspace_bytes returns the size with the full buffer. A smaller workspace (at
  * least the two-sweep size, which a too-small call names in its HM_ENOSPC message) gets a smaller buffer or none;
  * the outputs are the same, as they are when the buffer overflows (the columns then come from a second sweep).
@@ -156,8 +156,9 @@ int hm_pricing_norm(void* stream, const float* X, const float* Y, const double* 
 /*
  * hm_pricing_norm without a workspace and without any allocation. No counterpart in the reference: this entry
  * point is for callers that cannot allocate device memory (code under HIP graph capture, tight serving loops,
- * harnesses that forbid hipMalloc). Its scratch is a file-scope device array of hm_pricing_norm_noalloc_max_bytes()
- * bytes (64 MiB) per GPU, held until the process ends; calls whose two-sweep workspace exceeds it fail with HM_ENOSPC
+ * harnesses that forbid hipMalloc). Its scratch is a file-scope device array per GPU, held until the process ends, of
+ * hm_pricing_norm_noalloc_max_bytes() bytes (64 MiB) for the lists and some 1.4 MiB for what a call needs beside them; calls
+ * whose two-sweep workspace exceeds it fail with HM_ENOSPC
  * (524288 x 524288 at d = 8, k = 2 needs 12 MiB), and k <= 2 calls use the row sweep's column buffer only when all
  * of it fits (else two sweeps, same outputs). The scratch of the CURRENT device is used, so the
  * stream must belong to it. Every call on a GPU shares that GPU's array: calls that overlap on one GPU (other host
