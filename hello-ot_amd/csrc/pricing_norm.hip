@@ -1213,7 +1213,10 @@ int norm_direction_t(hipStream_t st, const Direction& D, int d, int k, const Nor
 // Entry floors of one side's lists (norm_seed) from 1/32 of the columns, at least 1024 of them: a floor then lets through
 // a few times the k pairs a list keeps on a short side. Short lists find the rest of the way themselves (at most 1024
 // columns: under a hundredth of the sweep on long sides); long ones take up to 4096. Split over enough workgroups to
-// fill the chip with at least 32 columns each.
+// fill the chip with at least 32 columns each. Where the rows alone fill it (256 workgroups) the sample's own time counts:
+// lists of up to 8 then take 1/16 of the columns of a short side, at least 128 (top-1 rows of l1, d = 5, 200000 x 1000 /
+// 3000 / 8000: 0.71 / 0.95 / 1.53 -> 0.38 / 0.72 / 1.37 ms; top-16 would go 4.5 -> 5.3 and 3000 x 3000 0.069 -> 0.089).
+constexpr int64_t SEED_FULL_ROWS = 65536;
 struct Seeding {
     const float* X;
     SweepSide side;
@@ -1226,7 +1229,9 @@ template <int KIND, int DR, bool TAIL>
 int norm_seed_t(hipStream_t st, const Seeding& s, int d, int k) {
     int64_t count = s.n / 32;
     const int64_t most = k <= 4 ? 1024 : 4096;
-    count = count < 1024 ? 1024 : (count > most ? most : count);
+    int64_t least = 1024;
+    if (s.m >= SEED_FULL_ROWS && k <= 8) least = s.n / 16 < 128 ? 128 : (s.n / 16 > 1024 ? 1024 : s.n / 16);
+    count = count < least ? least : (count > most ? most : count);
     if (count > s.n) count = s.n;
     const int64_t blocks = (s.m + 255) / 256;
     int64_t q = (1024 + blocks - 1) / blocks;

@@ -356,6 +356,24 @@ def test_norm_bidirectional_matches_oracle(cuda, kind, m, n, d, k):
 
 
 @pytest.mark.parametrize("kind", [0, 1, 2])
+@pytest.mark.parametrize("m,n,k", [(65535, 200, 2), (65536, 200, 8), (65537, 5, 8), (65536, 129, 9), (65793, 700, 1)])
+def test_norm_floors_of_many_rows_on_a_short_side(cuda, kind, m, n, k):
+    """From 65536 rows on, lists of up to 8 take their entry floors from fewer columns of a short side (its sixteenth part,
+    at least 128): the lists of both sides, alone and together, stay the oracle's bit for bit."""
+    rng = np.random.default_rng(m + n + k + kind)
+    X = rng.random((m, 5)).astype(np.float32)
+    Y = rng.random((n, 5)).astype(np.float32)
+    f = rng.normal(0.3, 0.2, m)
+    g = rng.normal(0.3, 0.2, n)
+    orv, ori, ocv, oci, ost = oracle.norm_scan(X, Y, f, g, k, kind)
+    rv, ri, cv, ci, st = pricing_norm(*_to(cuda, X, Y, f, g), k, kind)
+    av, ai, *_ = pricing_norm(*_to(cuda, X, Y, f, g), k, kind, cols=False, stats=False)
+    for got, want in ((ri, ori), (ci, oci), (rv, orv), (cv, ocv), (ai, ori), (av, orv)):
+        np.testing.assert_array_equal(got.cpu().numpy(), want)
+    _assert_stats(st, ost)
+
+
+@pytest.mark.parametrize("kind", [0, 1, 2])
 @pytest.mark.parametrize("m,n,d,k", [(300, 257, 8, 2), (129, 700, 3, 8), (64, 64, 40, 1), (20, 30, 100, 5),
                                      (257, 300, 64, 32), (40, 600, 130, 2)])
 def test_norm_fp64_bidirectional_matches_oracle(cuda, kind, m, n, d, k):
