@@ -1051,16 +1051,26 @@ inline NormPlan norm_segments(int64_t rows, int64_t cols, int64_t rows_per_block
 // The fp64 sweep: 256 threads, one row each. The fp32 sweep: two rows per thread share the loads and tests of a Y row
 // where their features fit the registers beside enough waves (d <= 32) and the problem still fills the chip. Its partial
 // lists take no more than those of one row per thread, or 24 MiB.
-// Lists in LDS, 12 k bytes a row, leave few waves on a CU (8 at k = 16, 6 at k = 32), too few for a pair loop of few
-// features; in their place in the partial lists, in memory, an entry costs more and a pair less. Top-16 (top-32) rows, l1, in
-// LDS and in memory, d = 8: 65536 x 65536 16.8 and 14.1 ms (55 and 43), 262144 x 262144 99 and 58 (273 and 120),
-// 524288 x 524288 379 and 200 (894 and 332); d = 32: 65536 x 65536 19.1 and 16.0. Lists of 5 to 8 are level at
-// 131072 x 131072 (13.3 and 13.7) and behind below (65536: 5.1 and 5.8); 180000 x 180000 32.1 and 20.8, 524288 x 524288 183
-// and, with two rows per thread, 128. Rows of more than 32 features keep LDS, with 128 threads for lists of more than 16.
+// Lists in LDS, 12 k bytes a row, leave few waves on a CU: 20 at k = 9 and 10, 12 to 16 at k = 11 to 16, 10 at k = 17 to 20
+// (128 threads from 17 on), 8 and 6 beyond. In their place in the partial lists, in memory, an entry costs more and a
+// pair less, so memory wins on long sides, and first where the waves in LDS are few for their k. Rows of l1, in LDS and in
+// memory, d = 8:
+//   k = 16: 16384^2 3.8 and 3.6 ms, 32768^2 9.1 and 8.1, 262144^2 99 and 58, 524288^2 379 and 200 (k = 11: 2.5 and 2.5,
+//           5.7 and 5.3; k = 14: 3.1 and 3.5, 7.3 and 7.7, 65536^2 14.0 and 13.4); both sides of 3000^2 1.15 and 1.45
+//   k = 32: 16384^2 13.4 and 9.5, 65536^2 56 and 44, 524288^2 894 and 332; both sides of 3000^2 2.2 and 2.9
+//   k = 9: 65536^2 5.8 and 7.0, 131072^2 14.2 and 15.4; k = 20: 65536^2 15.2 and 23.3, 131072^2 32 and 38
+//   k = 8: 65536^2 5.1 and 5.8, 131072^2 13.3 and 13.7, 180000^2 32.1 and 20.8, 524288^2 183 and, two rows a thread, 128.
+// Rows of more than 32 features keep LDS.
+inline bool lists_in_memory(int64_t rows, int64_t cols, int d, int k) {
+    if (d > GLOBAL_FEATURES || k <= 4 || (k <= 8 && d > 8)) return false;
+    const bool few_waves = (k > 10 && k <= 16) || k > 20;
+    return rows > (int64_t(1) << (few_waves ? 29 : 34)) / cols;
+}
+
 inline NormPlan norm_plan(int64_t rows, int64_t cols, int d, int k, uint32_t flags) {
     const NormPlan one = norm_segments(rows, cols, NB_ROWS, 64);
     if (flags & HM_FP64) return one;
-    const bool global = d <= GLOBAL_FEATURES && (k > 8 || (k > 4 && d <= 8 && rows > (int64_t(1) << 34) / cols));
+    const bool global = lists_in_memory(rows, cols, d, k);
     const int T = k > 16 && !global ? 128 : 256;
     const bool fills = ((rows + 511) / 512) * ((cols + NT - 1) / NT) >= 4096;
     const int R = d <= 32 && ((k <= 4 && fills) || (global && k <= 8 && rows >= 524288)) ? 2 : 1;

@@ -693,17 +693,19 @@ def test_norm_two_rows_per_thread_agree_with_one(cuda, kind, d, dense):
 
 
 @pytest.mark.parametrize("kind", [0, 1, 2])
-@pytest.mark.parametrize("m,n,d", [(140001, 130001, 7), (524288 + 77, 33001, 3)])
-def test_norm_lists_in_memory_agree_with_lists_in_lds(cuda, kind, m, n, d):
-    """Above 2^34 pairs lists of 5 to 8 entries lie in memory (with two rows per thread from 524288 rows on), as lists of
-    more than 8 do at any size; lists of 4 lie in LDS. Each holds the shorter one's entries first; the certificates differ
-    by the order of their sums (1e-9)."""
+@pytest.mark.parametrize("m,n,d,ks", [(140001, 130001, 7, (4, 8, 9)), (524288 + 77, 33001, 3, (4, 8, 9)),
+                                      (23100, 23101, 20, (10, 16, 32)), (23200, 23201, 20, (10, 11, 16, 17, 20, 21, 32)),
+                                      (200001, 2800, 32, (10, 13, 20, 24))])
+def test_norm_lists_in_memory_agree_with_lists_in_lds(cuda, kind, m, n, d, ks):
+    """Lists of 11 to 16 and of more than 20 entries lie in memory above 2^29 pairs, other lists of more than 4 (more than
+    8 past 8 features) above 2^34, with two rows per thread from 524288 rows on; the others lie in LDS. Each holds the
+    shorter one's entries first; the certificates differ by the order of their sums (1e-9)."""
     g0 = torch.Generator(device=cuda).manual_seed(7 + d)
     X = torch.rand(m, d, generator=g0, device=cuda)
     Y = torch.rand(n, d, generator=g0, device=cuda)
     f = 0.1 * torch.rand(m, generator=g0, device=cuda, dtype=torch.float64)
     g = 0.1 * torch.rand(n, generator=g0, device=cuda, dtype=torch.float64)
-    lists = [pricing_norm(X, Y, f, g, k, kind, cols=False) for k in (4, 8, 9)]
+    lists = [pricing_norm(X, Y, f, g, k, kind, cols=False) for k in ks]
     for short, long in zip(lists, lists[1:]):
         k = short[0].shape[1]
         assert torch.equal(short[0], long[0][:, :k]) and torch.equal(short[1], long[1][:, :k])
